@@ -70,7 +70,7 @@ def _compile(source: Path, flags: list[str]) -> Path:
 # operand addressing, and the product kernels a compiled epilogue is built
 # into.
 EMBEDDED = {"scalar_ops.h": "tc_scalar_ops_source", "device.hpp": "tc_device_source",
-            "gemm_kernels.hpp": "tc_gemm_kernels_source"}
+            "gemm_kernels.hpp": "tc_gemm_kernels_source", "gemm_sliced.hpp": "tc_gemm_sliced_source"}
 
 
 def _embedded_sources() -> Path:

@@ -206,6 +206,7 @@ bool dense_plan(const tc_encoded* code, uint32_t count, const tc_place* places, 
 extern "C" const char tc_scalar_ops_source[];
 extern "C" const char tc_device_source[];
 extern "C" const char tc_gemm_kernels_source[];
+extern "C" const char tc_gemm_sliced_source[];
 
 constexpr int kCompiledConstants = kInlineCode;
 
@@ -486,9 +487,10 @@ std::unordered_map<std::string, KernelResources> resources_by_function(const std
 // extern "C" name or a template-id whose lowered name hiprtc reports.
 bool compile_program(const std::string& source, const std::vector<std::string>& kernels, Compiled* out) {
     hiprtcProgram program;
-    const char* headers[] = {tc_scalar_ops_source, tc_device_source, tc_gemm_kernels_source};
-    const char* names[] = {"scalar_ops.h", "device.hpp", "gemm_kernels.hpp"};
-    if (hiprtcCreateProgram(&program, source.c_str(), "tc_fused_program.hip", 3, headers, names) != HIPRTC_SUCCESS) {
+    const char* headers[] = {tc_scalar_ops_source, tc_device_source, tc_gemm_kernels_source,
+                             tc_gemm_sliced_source};
+    const char* names[] = {"scalar_ops.h", "device.hpp", "gemm_kernels.hpp", "gemm_sliced.hpp"};
+    if (hiprtcCreateProgram(&program, source.c_str(), "tc_fused_program.hip", 4, headers, names) != HIPRTC_SUCCESS) {
         return false;
     }
     for (const std::string& kernel : kernels) {

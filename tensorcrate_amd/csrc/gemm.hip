@@ -29,10 +29,12 @@
 // steps, since the sum over k does not care which lane holds which k as long
 // as both operands agree.
 //
-// Operands whose rows are not 16-byte aligned, or past 2^31 bytes, take the
-// general kernels: both operands K-contiguous, one stored the other way round
-// first transposed into a scratch block, loads bounds-checked element by
-// element.
+// Products too small to give those tiles to most CUs, and operands whose rows
+// are not 16-byte aligned, take the register-fed kernel (gemm_sliced.hpp).
+//
+// Operands past 2^31 bytes take the general kernels: both operands
+// K-contiguous, one stored the other way round first transposed into a
+// scratch block, loads bounds-checked element by element.
 //
 // Block tiles are ordered in groups of rows, and the linear block index is
 // first spread so that the blocks one XCD runs are neighbours, which keeps
@@ -46,6 +48,7 @@
 
 #include "common.hpp"
 #include "gemm_kernels.hpp"
+#include "gemm_sliced.hpp"
 #include "program.hpp"
 
 namespace tc {
@@ -365,6 +368,58 @@ void launch_inplace32(const float* a, const float* b, O* c, uint32_t m, uint32_t
     inplace32_kernel<O, A_KC, B_KC, 128, 128, EPI><<<tiles, kThreads, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
 }
 
+// ---- register-fed products -----------------------------------------------------------
+//
+// The sliced kernel's tile for a product: 64 x 64 where that gives at least
+// half the CUs a block, else 32 x 32 where that does, else 16 x 16, and never
+// a tile twice the product's smaller side.  More, smaller tiles fill the chip
+// but read the operands more often (us a call): f32 768^3, 144 / 576 tiles of
+// 64 / 32: 17.7 / 20.0; f32 512^3, 64 / 256: 12.6 / 5.8; f32 256 x 8192 x 256,
+// 64 / 256 tiles of 32 / 16: 44 / 27; bf16 64 x 4096 x 4096 with B transposed,
+// 64 / 256 / 1024 of 64 / 32 / 16: 32 / 17 / 45.
+uint32_t sliced_tile(uint32_t m, uint32_t n) {
+    const uint64_t cus = static_cast<uint64_t>(compute_units());
+    const uint32_t narrow = std::min(m, n);
+    for (uint32_t tile = 64; tile > 16; tile /= 2) {
+        const uint64_t blocks = static_cast<uint64_t>((m + tile - 1) / tile) * ((n + tile - 1) / tile);
+        if (narrow > tile / 2 && blocks * 2 >= cus) return tile;
+    }
+    return 16;
+}
+
+// Whether a product whose operands the tiled kernels can read is small enough
+// for the sliced kernel instead.  A tiled 16-bit block does a 64-deep step in
+// about 0.8 us whether or not the other CUs have a tile, while the sliced
+// kernel runs at 300-320 TFLOP/s on these: they meet near half a 128 x 128
+// tile a CU (us a call, tiled / sliced: 64 tiles, 1024^3, 14.8 / 9.3; 192,
+// 2048 x 1024 x 1536, 15.5 / 21.8).  f32's matrix cores are sixteen times
+// slower, so the sliced kernel's extra reads hide for longer: 64 tiles
+// 44.9 / 22.4, 192 tiles 71.7 / 73.
+bool small_product(uint32_t m, uint32_t n, bool f32) {
+    const uint64_t tiles = static_cast<uint64_t>((m + 127) / 128) * ((n + 127) / 128);
+    return tiles * 4 < static_cast<uint64_t>(compute_units()) * (f32 ? 3 : 2);
+}
+
+// The sliced kernel addresses its operands with 32-bit byte offsets.
+bool sliced_reach(uint64_t m, uint64_t k, uint64_t n, size_t width) {
+    const uint64_t limit = uint64_t{1} << 31;
+    return m * k * width < limit && k * n * width < limit;
+}
+
+template <typename S, typename O, bool A_KC, bool B_KC, class EPI = PlainStore>
+void launch_sliced(const S* a, const S* b, O* c, uint32_t m, uint32_t k, uint32_t n, bool accumulate, hipStream_t s,
+                   const EPI& epi = EPI{}) {
+    const uint32_t tile = sliced_tile(m, n);
+    const uint32_t blocks = ((m + tile - 1) / tile) * ((n + tile - 1) / tile);
+    if (tile == 64) {
+        sliced_kernel<S, O, A_KC, B_KC, 4, 4, 4, 1, EPI><<<blocks, 256, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
+    } else if (tile == 32) {
+        sliced_kernel<S, O, A_KC, B_KC, 2, 2, 4, 1, EPI><<<blocks, 256, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
+    } else {
+        sliced_kernel<S, O, A_KC, B_KC, 1, 1, 8, 4, EPI><<<blocks, 512, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
+    }
+}
+
 // ---- products over a short K -----------------------------------------------------------
 //
 // A product with K below 8 (an outer product, K = 1, is how the tape
@@ -488,17 +543,27 @@ int matmul_typed(uint32_t transposed, bool accumulate, uint64_t m, uint64_t k, u
         if (transposed == TC_LEFT) return launch_short_k<S, O, false, false>(pa, pb, pc, m, k, n, accumulate, s);
         return launch_short_k<S, O, true, true>(pa, pb, pc, m, k, n, accumulate, s);
     }
-    if constexpr (std::is_same<S, float>::value) {
-        // f32 operands read in place whenever their rows are 16-byte aligned
-        // and they stay under the buffer offsets' 2^31 bytes.
-        const bool a_kc = transposed != TC_LEFT, b_kc = transposed == TC_RIGHT;
-        const uint64_t limit = uint64_t{1} << 31;
-        const bool in_place = aligned16(a) && aligned16(b) && (a_kc ? k % 4 == 0 : m % 4 == 0) &&
-                              (b_kc ? k % 4 == 0 : n % 4 == 0) && m * k * 4 < limit && k * n * 4 < limit;
-        if (in_place) {
-            const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k),
-                           n32 = static_cast<uint32_t>(n);
-            O* pc = static_cast<O*>(c);
+    // The tiled kernels read operands in place whenever their rows are 16-byte
+    // aligned (A is K-contiguous unless LEFT, B only when RIGHT) and stay
+    // under the buffer offsets' 2^31 bytes; small products, and other
+    // operands, take the register-fed kernel.
+    const bool a_kc = transposed != TC_LEFT, b_kc = transposed == TC_RIGHT;
+    constexpr uint64_t kRun = 16 / sizeof(S);
+    const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
+    if (sliced_reach(m, k, n, sizeof(S))) {
+        O* pc = static_cast<O*>(c);
+        const bool in_place = aligned16(a) && aligned16(b) && (a_kc ? k : m) % kRun == 0 && (b_kc ? k : n) % kRun == 0;
+        if (!in_place || small_product(m32, n32, std::is_same<S, float>::value)) {
+            if (a_kc && b_kc) {
+                launch_sliced<S, O, true, true>(pa, pb, pc, m32, k32, n32, accumulate, s);
+            } else if (a_kc) {
+                launch_sliced<S, O, true, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
+            } else {
+                launch_sliced<S, O, false, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
+            }
+            return check_launch("matmul");
+        }
+        if constexpr (std::is_same<S, float>::value) {
             if (a_kc && b_kc) {
                 launch_inplace32<O, true, true>(pa, pb, pc, m32, k32, n32, accumulate, s);
             } else if (a_kc) {
@@ -506,22 +571,7 @@ int matmul_typed(uint32_t transposed, bool accumulate, uint64_t m, uint64_t k, u
             } else {
                 launch_inplace32<O, false, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
             }
-            return check_launch("matmul");
-        }
-    } else {
-        // 16-bit operands read in place whenever their rows are 16-byte
-        // aligned: A is K-contiguous unless LEFT, B only when RIGHT.
-        const bool a_kc = transposed != TC_LEFT, b_kc = transposed == TC_RIGHT;
-        // The tiled kernel addresses each operand with 32-bit buffer offsets
-        // and points the K tail past 2^31 bytes, so operands stay below it.
-        const uint64_t limit = uint64_t{1} << 31;
-        const bool in_place = aligned16(a) && aligned16(b) && (a_kc ? k % 8 == 0 : m % 8 == 0) &&
-                              (b_kc ? k % 8 == 0 : n % 8 == 0) && m * k * sizeof(S) < limit &&
-                              k * n * sizeof(S) < limit;
-        if (in_place) {
-            const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k),
-                           n32 = static_cast<uint32_t>(n);
-            O* pc = static_cast<O*>(c);
+        } else {
             if (a_kc && b_kc) {
                 launch_tiled16<S, O, true, true>(pa, pb, pc, m32, k32, n32, accumulate, s);
             } else if (a_kc) {
@@ -529,8 +579,8 @@ int matmul_typed(uint32_t transposed, bool accumulate, uint64_t m, uint64_t k, u
             } else {
                 launch_tiled16<S, O, false, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
             }
-            return check_launch("matmul");
         }
+        return check_launch("matmul");
     }
     void* made_a = nullptr;
     void* made_b = nullptr;
@@ -564,8 +614,9 @@ constexpr int kCompiledElems = 16;
 // after the product kernels' header; empty when the program has more
 // constants than the kernels' arguments carry.
 std::string epilogue_source(uint32_t dtype, const tc_encoded* code, uint32_t count, const tc_place* host_places,
-                            std::vector<float>* constants, bool runs, bool* has_runs = nullptr) {
-    const std::string body = epilogue_group(code, count, dtype, true, kCompiledElems, host_places, constants);
+                            std::vector<float>* constants, bool runs, bool* has_runs = nullptr,
+                            int elems = kCompiledElems, const char* header = "gemm_kernels.hpp") {
+    const std::string body = epilogue_group(code, count, dtype, true, elems, host_places, constants);
     // The run form, where the operands allow it (the caller's `runs`): runs
     // of eight for the four-wave kernel's 16-bit products, of four for the
     // f32 kernel.
@@ -574,15 +625,60 @@ std::string epilogue_source(uint32_t dtype, const tc_encoded* code, uint32_t cou
              : std::string();
     if (constants->size() > static_cast<size_t>(kInlineCode)) return std::string();
     if (has_runs != nullptr) *has_runs = !run_members.empty();
-    return "#include \"gemm_kernels.hpp\"\n"
+    return std::string("#include \"") + header + "\"\n"
            "struct CompiledStore {\n"
            "  static constexpr bool kProgram = true;\n"
            "  static constexpr bool kRuns = " + std::string(run_members.empty() ? "false" : "true") + ";\n"
-           "  static constexpr int kElems = " + std::to_string(kCompiledElems) + ";\n" +
+           "  static constexpr int kElems = " + std::to_string(elems) + ";\n" +
            compiled_members() +
            "  __device__ __forceinline__ void group(const bool (&live)[kElems], const uint32_t (&row)[kElems],\n"
            "      const uint32_t (&col)[kElems], uint32_t N, const float (&product)[kElems]) const {\n" +
            body + "  }\n" + run_members + "};\n";
+}
+
+// The arguments of a compiled epilogue's program.
+CompiledArgsOf compiled_args(const std::vector<float>& constants, const DevicePlace* places, uint32_t place_count,
+                             const void* const* inputs, uint32_t input_count, void* const* outputs,
+                             uint32_t output_count) {
+    CompiledArgsOf args{};
+    for (uint32_t slot = 1; slot < input_count; slot++) args.in[slot] = inputs[slot];
+    for (uint32_t slot = 0; slot < output_count; slot++) args.out[slot] = outputs[slot];
+    for (uint32_t p = 0; p < place_count; p++) args.places[p] = places[p];
+    for (size_t c = 0; c < constants.size(); c++) args.constants[c] = constants[c];
+    return args;
+}
+
+// The sliced kernel of this product's tile with `code` compiled into its
+// epilogue, as `run_compiled_epilogue` does for the tiled kernels: each lane
+// finishes its 4 values of each 16 x 16 tile across, all at once.
+bool run_compiled_sliced(uint32_t dtype, uint32_t m, uint32_t k, uint32_t n, const void* a, const void* b,
+                         const tc_encoded* code, uint32_t count, const tc_place* host_places,
+                         const DevicePlace* places, uint32_t place_count, const void* const* inputs,
+                         uint32_t input_count, void* const* outputs, uint32_t output_count, hipStream_t s,
+                         int* status) {
+    const uint32_t tile = sliced_tile(m, n);
+    const std::string type = dtype == TC_F32 ? "float" : dtype == TC_F16 ? "_Float16" : "tc::bf16_t";
+    const std::string shape = tile == 64 ? "4, 4, 4, 1" : tile == 32 ? "2, 2, 4, 1" : "1, 1, 8, 4";
+    std::vector<float> constants;
+    const std::string source = epilogue_source(dtype, code, count, host_places, &constants, false, nullptr,
+                                               static_cast<int>(tile / 4), "gemm_sliced.hpp");
+    if (source.empty()) return false;
+    hipFunction_t function = nullptr;
+    KernelResources resources;
+    if (!compiled_kernels(source, {"tc::sliced_kernel<" + type + ", " + type + ", true, false, " + shape +
+                                   ", CompiledStore>"}, &function, &resources)) {
+        return false;
+    }
+    CompiledArgsOf args = compiled_args(constants, places, place_count, inputs, input_count, outputs, output_count);
+    void* none = nullptr;
+    bool accumulate = false;
+    void* params[] = {const_cast<void**>(&a), const_cast<void**>(&b), &none, &m, &n, &k, &accumulate, &args};
+    const uint32_t blocks = ((m + tile - 1) / tile) * ((n + tile - 1) / tile);
+    count_dispatch();
+    const hipError_t error =
+        hipModuleLaunchKernel(function, blocks, 1, 1, tile == 16 ? 512 : 256, 1, 1, 0, s, params, nullptr);
+    *status = error == hipSuccess ? TC_OK : fail(TC_DEVICE, std::string("fused matmul: ") + hipGetErrorString(error));
+    return true;
 }
 
 // The most architectural VGPRs a four-wave instance with a compiled
@@ -631,11 +727,7 @@ bool run_compiled_epilogue(uint32_t dtype, uint32_t m, uint32_t k, uint32_t n, c
     hipFunction_t functions[4] = {};
     KernelResources resources[4];
     if (!compiled_kernels(source, kernels, functions, resources)) return false;
-    CompiledArgsOf args{};
-    for (uint32_t slot = 1; slot < input_count; slot++) args.in[slot] = inputs[slot];
-    for (uint32_t slot = 0; slot < output_count; slot++) args.out[slot] = outputs[slot];
-    for (uint32_t p = 0; p < place_count; p++) args.places[p] = places[p];
-    for (size_t c = 0; c < constants.size(); c++) args.constants[c] = constants[c];
+    CompiledArgsOf args = compiled_args(constants, places, place_count, inputs, input_count, outputs, output_count);
     void* none = nullptr;
     bool accumulate = false;
     void* params[] = {const_cast<void**>(&a), const_cast<void**>(&b), &none, &m, &n, &k, &accumulate, &args};
@@ -687,13 +779,17 @@ int matmul_program(uint32_t dtype, uint64_t m, uint64_t k, uint64_t n, const voi
     }
     TC_STREAM(s);
     const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
+    // The kernel `tc_matmul` takes for this product, so that the program sees
+    // the same bits.
+    const bool small = small_product(m32, n32, dtype == TC_F32);
     int status = TC_OK;
     {
         DevicePlace device_places[kInlinePlaces] = {};
         status = to_device_places(places, place_count, device_places);
         if (status != TC_OK) return status;
-        if (run_compiled_epilogue(dtype, m32, k32, n32, a, b, code, count, places, device_places, place_count, inputs,
-                                  input_count, outputs, output_count, s, &status)) {
+        const auto run_compiled = small ? run_compiled_sliced : run_compiled_epilogue;
+        if (run_compiled(dtype, m32, k32, n32, a, b, code, count, places, device_places, place_count, inputs,
+                         input_count, outputs, output_count, s, &status)) {
             *fused = true;
             return status;
         }
@@ -706,31 +802,26 @@ int matmul_program(uint32_t dtype, uint64_t m, uint64_t k, uint64_t n, const voi
         epi.count = count;
         return status == TC_OK;
     };
+    auto launch = [&](auto epi, auto element) {
+        using S = decltype(element);
+        if (!interpreted(epi)) return;
+        const S *pa = static_cast<const S*>(a), *pb = static_cast<const S*>(b);
+        S* none = nullptr;
+        if (small) {
+            launch_sliced<S, S, true, false>(pa, pb, none, m32, k32, n32, false, s, epi);
+        } else if constexpr (std::is_same<S, float>::value) {
+            launch_inplace32<S, true, false>(pa, pb, none, m32, k32, n32, false, s, epi);
+        } else {
+            launch_tiled16<S, S, true, false>(pa, pb, none, m32, k32, n32, false, s, epi);
+        }
+    };
     switch (dtype) {
-        case TC_F32: {
-            ProgramStore<TC_F32> epi{};
-            if (!interpreted(epi)) return status;
-            launch_inplace32<float, true, false>(static_cast<const float*>(a), static_cast<const float*>(b), nullptr,
-                                                 m32, k32, n32, false, s, epi);
-            break;
-        }
-        case TC_F16: {
-            ProgramStore<TC_F16> epi{};
-            if (!interpreted(epi)) return status;
-            launch_tiled16<_Float16, _Float16, true, false>(static_cast<const _Float16*>(a),
-                                                            static_cast<const _Float16*>(b), nullptr, m32, k32, n32,
-                                                            false, s, epi);
-            break;
-        }
-        case TC_BF16: {
-            ProgramStore<TC_BF16> epi{};
-            if (!interpreted(epi)) return status;
-            launch_tiled16<bf16_t, bf16_t, true, false>(static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(b),
-                                                        nullptr, m32, k32, n32, false, s, epi);
-            break;
-        }
+        case TC_F32: launch(ProgramStore<TC_F32>{}, float{}); break;
+        case TC_F16: launch(ProgramStore<TC_F16>{}, _Float16{}); break;
+        case TC_BF16: launch(ProgramStore<TC_BF16>{}, bf16_t{}); break;
         default: return TC_OK;
     }
+    if (status != TC_OK) return status;
     *fused = true;
     return check_launch("fused matmul");
 }
