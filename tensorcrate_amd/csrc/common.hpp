@@ -283,6 +283,22 @@ __device__ __forceinline__ uint4 load_word(const void* p) {
     return *static_cast<const uint4*>(p);
 }
 
+// The same from any address: gfx950 loads words unaligned, one instruction
+// either way, so rows that start off 16 bytes need no path of their own.
+typedef uint32_t u32x4_anywhere __attribute__((ext_vector_type(4), aligned(1)));
+
+template <bool NT>
+__device__ __forceinline__ uint4 load_any_word(const void* p) {
+    const u32x4_anywhere* at = static_cast<const u32x4_anywhere*>(p);
+    u32x4 v;
+    if (NT) {
+        v = __builtin_nontemporal_load(at);
+    } else {
+        v = *at;
+    }
+    return uint4{v.x, v.y, v.z, v.w};
+}
+
 template <bool NT>
 __device__ __forceinline__ void store_word(void* p, uint4 v) {
     if (NT) {

@@ -15,17 +15,20 @@
 // NaNs never win, and a slice of NaNs answers index 0 (strided.rs:186-225).
 //
 // The host coalesces the kept and the folded axes separately and picks:
-//  - rows: the folded axes are one contiguous run; one wave per slice, lanes
-//    reading 16 bytes at a time, combined by a 64-lane shuffle tree;
+//  - rows: the folded axes are one contiguous run; a wave's lanes, or fewer
+//    for a short run, read it 16 bytes at a time and are combined by a shuffle
+//    tree;
 //  - columns: the innermost kept axis is contiguous and the folded axes are
-//    one strided axis; lanes take neighbouring columns so each row read is
-//    coalesced, four row groups split the depth inside a block, and long
-//    depths split across blocks, each result's splits then merged by one
-//    wave in a fixed order;
+//    one strided axis; lanes take neighbouring 16 bytes of columns so each row
+//    read is coalesced, and the rest of the block takes other rows;
 //  - general: one thread per slice walking its elements in row-major order.
+// The first two split a long depth over blocks where there are few results,
+// each result's splits then merged in a fixed order by a second kernel.  Both
+// read rows wherever they start.
 
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 #include <unordered_map>
 
@@ -47,6 +50,7 @@ namespace {
 template <uint32_t OP>
 struct Fold {
     using State = float;
+    static constexpr bool kLight = true;  // an instruction or two an element
     __device__ static State init() {
         return OP == TC_REDUCE_SUM ? 0.0f : (OP == TC_REDUCE_MIN ? INFINITY : -INFINITY);
     }
@@ -65,6 +69,17 @@ struct Fold {
     template <int U, int V>
     __device__ static void add_packs(State& s, const float (&x)[U * V], uint32_t, uint32_t) {
         add_chunk(s, x, 0);
+    }
+    // The first `left` of them, at least one.
+    template <int U, int V>
+    __device__ static void add_some(State& s, const float (&x)[U * V], uint32_t left, uint32_t, uint32_t) {
+        State c = init();
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+#pragma unroll
+            for (int j = 0; j < V; j++) c = static_cast<uint32_t>(k) < left ? combine(c, x[k * V + j]) : c;
+        }
+        s = combine(s, c);
     }
     __device__ static State merge(State a, State b) { return combine(a, b); }
     __device__ static State shuffle(State s, int lane) { return __shfl(s, lane, 64); }
@@ -86,6 +101,7 @@ __device__ inline Moments merge_moments(Moments a, Moments b) {
 
 struct Var {
     using State = Moments;
+    static constexpr bool kLight = false;
     __device__ static State init() { return Moments{0.0f, 0.0f, 0.0f}; }
     __device__ static void add(State& s, float x, uint32_t) { s = merge_moments(s, Moments{1.0f, x, 0.0f}); }
     // A chunk's own moments are exact two-pass ones from registers.
@@ -109,6 +125,21 @@ struct Var {
     __device__ static void add_packs(State& s, const float (&x)[U * V], uint32_t, uint32_t) {
         add_chunk(s, x, 0);
     }
+    template <int U, int V>
+    __device__ static void add_some(State& s, const float (&x)[U * V], uint32_t left, uint32_t, uint32_t) {
+        const float n = static_cast<float>(left * V);
+        float total = 0.0f;
+#pragma unroll
+        for (int k = 0; k < U * V; k++) total += static_cast<uint32_t>(k / V) < left ? x[k] : 0.0f;
+        const float mean = total / n;
+        float m2 = 0.0f;
+#pragma unroll
+        for (int k = 0; k < U * V; k++) {
+            const float d = static_cast<uint32_t>(k / V) < left ? x[k] - mean : 0.0f;
+            m2 += d * d;
+        }
+        s = merge_moments(s, Moments{n, mean, m2});
+    }
     __device__ static State merge(State a, State b) { return merge_moments(a, b); }
     __device__ static State shuffle(State s, int lane) {
         return Moments{__shfl(s.n, lane, 64), __shfl(s.mean, lane, 64), __shfl(s.m2, lane, 64)};
@@ -126,6 +157,7 @@ struct Arg {
 template <uint32_t OP>
 struct ArgFold {
     using State = Arg;
+    static constexpr bool kLight = false;
     __device__ static State init() { return Arg{NAN, 0u}; }
     __device__ static bool better(Arg b, Arg a) {
         if (isnan(b.value)) return false;
@@ -148,6 +180,16 @@ struct ArgFold {
         for (int k = 0; k < U; k++) {
 #pragma unroll
             for (int j = 0; j < V; j++) add(s, x[k * V + j], first + k * step + j);
+        }
+    }
+    template <int U, int V>
+    __device__ static void add_some(State& s, const float (&x)[U * V], uint32_t left, uint32_t first, uint32_t step) {
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                if (static_cast<uint32_t>(k) < left) add(s, x[k * V + j], first + k * step + j);
+            }
         }
     }
     __device__ static State merge(State a, State b) { return better(b, a) ? b : a; }
@@ -205,11 +247,12 @@ struct Finisher<ArgFold<OP>> {
     __device__ static void write(const Arg& s, const Finish&, uint32_t* out, uint64_t at) { out[at] = s.index; }
 };
 
+// The states of each `lanes` neighbouring lanes (a power of two up to 64).
 template <typename P>
-__device__ inline typename P::State wave_reduce(typename P::State s) {
+__device__ inline typename P::State wave_reduce(typename P::State s, int lanes = 64) {
     const int lane = threadIdx.x % 64;
 #pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) {
+    for (int offset = lanes / 2; offset > 0; offset >>= 1) {
         typename P::State other = P::shuffle(s, lane ^ offset);
         // The lower lane's state is the left operand, so the tree's order is
         // fixed and the result deterministic.
@@ -221,25 +264,23 @@ __device__ inline typename P::State wave_reduce(typename P::State s) {
 // The wave's moments in closed form rather than by six pairwise merges:
 // with N = sum n_i and mean = sum n_i mean_i / N,
 //     M2 = sum (M2_i + n_i (mean_i - mean)^2),
-// the identity each of Chan's merges applies, taken over all 64 lanes at
+// the identity each of Chan's merges applies, taken over all the lanes at
 // once.  Two shuffle-sum trees and one division instead of six divisions
 // and eighteen shuffles; the fixed tree keeps the result deterministic.
 // A butterfly sum: every lane ends with the same total (each step adds one
 // pair, and addition is commutative).
-__device__ inline float wave_sum(float v) {
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
+__device__ inline float wave_sum(float v, int lanes) {
+    for (int offset = lanes / 2; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
     return v;
 }
 
 template <>
-__device__ inline Moments wave_reduce<Var>(Moments s) {
-    const float n = wave_sum(s.n);
-    if (n == 0.0f) return Var::init();
-    const float mean = wave_sum(s.n * s.mean) / n;
+__device__ inline Moments wave_reduce<Var>(Moments s, int lanes) {
+    const float n = wave_sum(s.n, lanes);
+    const float mean = wave_sum(s.n * s.mean, lanes) / n;
     const float d = s.mean - mean;
-    const float m2 = wave_sum(s.n == 0.0f ? 0.0f : s.m2 + s.n * d * d);
-    return Moments{n, mean, m2};
+    const float m2 = wave_sum(s.n == 0.0f ? 0.0f : s.m2 + s.n * d * d, lanes);
+    return n == 0.0f ? Var::init() : Moments{n, mean, m2};
 }
 
 // ---- layouts ----------------------------------------------------------------
@@ -277,15 +318,19 @@ struct alignas(16) Pack {
     S v[N];
 };
 
-// ---- rows: one wave per contiguous slice ------------------------------------
+// ---- rows: a wave's lanes, or a few of them, per contiguous slice ------------
 
-// U packs of one lane, 64 packs apart, loaded together and widened.
-template <typename S, int U, bool NT>
-__device__ __forceinline__ void load_packs(const Pack<S>* packs, float (&x)[U * Pack<S>::N]) {
+// U packs of one lane from `pack` on, `apart` packs apart, loaded together and
+// widened; with EDGE the ones past pack `last` repeat it.
+template <typename S, int U, bool NT, bool EDGE, typename I>
+__device__ __forceinline__ void load_packs(const S* slice, I pack, I apart, I last, float (&x)[U * Pack<S>::N]) {
     constexpr int V = Pack<S>::N;
     uint4 w[U];
 #pragma unroll
-    for (int k = 0; k < U; k++) w[k] = load_word<NT>(packs + k * 64);
+    for (int k = 0; k < U; k++) {
+        const I at = pack + k * apart;
+        w[k] = load_any_word<NT>(slice + (EDGE && at > last ? last : at) * V);
+    }
 #pragma unroll
     for (int k = 0; k < U; k++) {
         Pack<S> p;
@@ -295,45 +340,85 @@ __device__ __forceinline__ void load_packs(const Pack<S>* packs, float (&x)[U * 
     }
 }
 
+// The rows' layout: `results` contiguous slices of `depth` elements, each cut
+// into `splits` of `per_split` (the last may hold fewer), `lanes` lanes (a
+// power of two up to 64) to a cut.
+template <typename I>
+struct RowWalk {
+    Kept<I> kept;
+    I results, depth;
+    I splits, per_split;
+    Div<I> splits_div;
+    uint32_t lanes;
+};
+
+// Bound by loads in flight.  Each lane has four packs in flight, so a slice
+// takes a quarter as many lanes as it has packs: a whole wave from 4 KiB, and
+// below that the wave takes several slices at once, which also shares the
+// shuffle tree and its shorter part of it between them.  Slices are read as
+// packs wherever they start, and a last group of fewer packs is loaded
+// together too.  us a call, before (a wave a slice, element by element where
+// 16 bytes did not divide the rows) / this, the launch included: bf16
+// [11550 x 513] sums 8.1 / 3.8, variances 10.6 / 4.7; f32 [10000 x 60] 8.9 /
+// 3.8; f32 [1 x 2000000], one wave before, 592 / 7.9; f32 [8192 x 1024], a
+// whole wave either way, 6.7 / 6.7.
+// MODE: a few lanes a slice, a whole wave, or a whole wave on a cut of one.
 // With NT the input streams past the Infinity Cache (inputs larger than it).
-template <typename S, typename P, typename O, bool PACKED, bool NT, typename I>
+enum class Rows { few, whole, split };
+template <typename S, typename P, typename O, Rows MODE, bool NT, typename I>
 __global__ void __launch_bounds__(256) rows_kernel(const S* __restrict__ in, O* __restrict__ out,
-                                                   Kept<I> kept, I results, I depth, Finish f) {
+                                                   typename P::State* __restrict__ partial, RowWalk<I> w, Finish f) {
     using E = Elem<S>;
     constexpr int V = Pack<S>::N;
-    // Four 16-byte packs in flight per lane: a 4 KiB row per wave at once.
     constexpr int U = 4;
-    const int lane = threadIdx.x % 64;
-    const I waves = static_cast<I>(gridDim.x) * (blockDim.x / 64);
-    for (I r = static_cast<I>(blockIdx.x) * (blockDim.x / 64) + threadIdx.x / 64; r < results; r += waves) {
-        const S* slice = in + kept_offset(kept, r);
+    const uint32_t lane = threadIdx.x % 64;
+    const uint32_t across = MODE == Rows::few ? w.lanes : 64;
+    const I lanes = across, at = lane & (across - 1);
+    const I per_wave = 64 / across, within = lane / across;
+    const I items = MODE == Rows::split ? w.results * w.splits : w.results;
+    const I stride = static_cast<I>(gridDim.x) * 4 * per_wave;
+    for (I base = (static_cast<I>(blockIdx.x) * 4 + threadIdx.x / 64) * per_wave; base < items; base += stride) {
+        const I item = base + within;
         typename P::State s = P::init();
-        if (PACKED) {
-            const Pack<S>* packs = reinterpret_cast<const Pack<S>*>(slice);
-            const I count = depth / V;
-            I p = lane;
-            for (; p + 64 * (U - 1) < count; p += 64 * U) {
+        I result = item;
+        if (item < items) {
+            I begin = 0, count = w.depth;
+            if constexpr (MODE == Rows::split) {
+                result = w.splits_div.div(item);
+                begin = (item - result * w.splits) * w.per_split;
+                count = w.depth - begin < w.per_split ? w.depth - begin : w.per_split;
+            }
+            const S* slice = in + kept_offset(w.kept, result) + begin;
+            const I packs = count / V;
+            I p = at;
+            for (; p + lanes * (U - 1) < packs; p += lanes * U) {
                 float x[U * V];
-                load_packs<S, U, NT>(packs + p, x);
-                P::template add_packs<U, V>(s, x, static_cast<uint32_t>(p * V), 64 * V);
+                load_packs<S, U, NT, false, I>(slice, p, lanes, 0, x);
+                P::template add_packs<U, V>(s, x, static_cast<uint32_t>(begin + p * V), static_cast<uint32_t>(lanes * V));
             }
-            for (; p < count; p += 64) {
-                float x[V];
-                load_packs<S, 1, NT>(packs + p, x);
-                P::template add_packs<1, V>(s, x, static_cast<uint32_t>(p * V), 0);
+            if (p < packs) {
+                float x[U * V];
+                load_packs<S, U, NT, true, I>(slice, p, lanes, packs - 1, x);
+                const uint32_t left = static_cast<uint32_t>((packs - p + lanes - 1) / lanes);
+                P::template add_some<U, V>(s, x, left, static_cast<uint32_t>(begin + p * V),
+                                           static_cast<uint32_t>(lanes * V));
             }
-        } else {
-            for (I i = lane; i < depth; i += 64) P::add(s, E::widen(slice[i]), static_cast<uint32_t>(i));
+            for (I i = packs * V + at; i < count; i += lanes) {
+                P::add(s, E::widen(slice[i]), static_cast<uint32_t>(begin + i));
+            }
         }
-        s = wave_reduce<P>(s);
-        if (lane == 0) Finisher<P>::write(s, f, out, r);
+        s = wave_reduce<P>(s, static_cast<int>(across));
+        if (at == 0 && item < items) {
+            if constexpr (MODE == Rows::split) {
+                partial[item] = s;
+            } else {
+                Finisher<P>::write(s, f, out, result);
+            }
+        }
     }
 }
 
 // ---- columns: lanes on neighbouring kept columns ----------------------------
-
-constexpr int kColumns = 64;
-constexpr int kGroups = 4;
 
 // The columns' layout: results are [outer, columns] with the columns
 // contiguous in the input; each column folds `depth` elements `step` apart.
@@ -346,23 +431,80 @@ struct ColumnWalk {
     Div<I> tiles_div;
     I splits;       // depth splits across blocks
     I per_split;    // rows per split (the last may hold fewer)
+    uint32_t lanes;   // lanes across a tile's columns
+    uint32_t groups;  // row groups: lanes x groups is at most a block's 256
+    bool apart;       // a group's rows are `groups` apart rather than a run of them
+    DivMod lanes_div;
 };
 
-// One block: kColumns lanes, each on VC neighbouring columns (VC > 1 reads
-// them as one 16-byte word), times kGroups row groups over one split's rows.
-// With splits == 1 it finishes the results; otherwise it writes its states
-// to `partial[result * splits + split]` for the combine kernels.
-template <typename S, typename P, typename O, int VC, bool NT, typename I>
+// VC neighbouring columns of one row, 16 bytes of them or 4, wherever they start.
+template <bool NT, typename S, int VC>
+__device__ __forceinline__ void load_columns(const S* at, S (&v)[VC]) {
+    if constexpr (sizeof(S) * VC == 16) {
+        const uint4 word = load_any_word<NT>(at);
+        __builtin_memcpy(v, &word, 16);
+    } else {
+        __builtin_memcpy(v, at, sizeof(v));
+    }
+}
+
+// The states of a block's groups merged into group 0's, in a fixed order:
+// thread group * lanes + lane holds VC states.  Up to four groups meet at once;
+// more (narrow rows) first halve, a pair a step.
+template <typename P, int VC>
+__device__ __forceinline__ void merge_groups(typename P::State (&s)[VC], typename P::State (*stage)[256],
+                                             uint32_t group, uint32_t groups, uint32_t lanes) {
+    while (groups > 4) {
+        const uint32_t half = (groups + 1) / 2;
+        if (group >= half) {
+#pragma unroll
+            for (int c = 0; c < VC; c++) stage[c][threadIdx.x] = s[c];
+        }
+        __syncthreads();
+        if (group + half < groups) {
+#pragma unroll
+            for (int c = 0; c < VC; c++) s[c] = P::merge(s[c], stage[c][threadIdx.x + half * lanes]);
+        }
+        __syncthreads();
+        groups = half;
+    }
+    if (group > 0) {
+#pragma unroll
+        for (int c = 0; c < VC; c++) stage[c][threadIdx.x] = s[c];
+    }
+    __syncthreads();
+    if (group == 0) {
+        for (uint32_t g = 1; g < groups; g++) {
+#pragma unroll
+            for (int c = 0; c < VC; c++) s[c] = P::merge(s[c], stage[c][threadIdx.x + g * lanes]);
+        }
+    }
+    __syncthreads();
+}
+
+// One block: `lanes` lanes on VC neighbouring columns each (one word, wherever
+// it starts; a last word that would pass the columns starts earlier and its
+// first columns are not written; at least VC columns), times
+// `groups` row groups sharing one split's rows, eight rows in flight a lane.
+// With splits == 1 it finishes the results; otherwise it writes its states to
+// `partial[result * splits + split]` for the combine kernels.
+// Bound by loads in flight and by how evenly the columns fill the lanes.  WIDE:
+// 64 lanes, four groups, each a run of rows.  us a call with its launches,
+// before (64 lanes, one column each; under 16 columns a thread a result) /
+// this: bf16 [60480 x 11] sums 7877 / 6.3, [11550 x 513] 9.5 / 8.6; f32
+// [14688 x 11] 1700 / 6.3, [8192 x 1024] 9.0 / 9.0.
+template <typename S, typename P, typename O, int VC, bool WIDE, bool NT, typename I>
 __global__ void __launch_bounds__(256) columns_kernel(const S* __restrict__ in, O* __restrict__ out,
                                                       typename P::State* __restrict__ partial,
                                                       ColumnWalk<I> w, I blocks, Finish f) {
     using E = Elem<S>;
     using State = typename P::State;
-    // Rows in flight per lane.
     constexpr int U = 8;
-    __shared__ State stage[kGroups][VC][kColumns];
-    const int lane = threadIdx.x % kColumns;
-    const int group = threadIdx.x / kColumns;
+    __shared__ State stage[VC][256];
+    const uint32_t lanes = WIDE ? 64 : w.lanes, groups = WIDE ? 4 : w.groups;
+    const bool apart = !WIDE && w.apart;
+    const uint32_t group = WIDE ? threadIdx.x / 64 : w.lanes_div.div(threadIdx.x);
+    const uint32_t lane = threadIdx.x - group * lanes;
     for (I block = blockIdx.x; block < blocks; block += gridDim.x) {
         // block -> (split, outer, tile), split outermost so neighbouring
         // blocks share rows.
@@ -371,76 +513,61 @@ __global__ void __launch_bounds__(256) columns_kernel(const S* __restrict__ in, 
         const I rest = block - split * per_split_blocks;
         const I outer = w.tiles_div.div(rest);
         const I tile = rest - outer * w.tiles;
-        // With VC > 1 the columns are a multiple of VC, so a lane's first
-        // column in range puts all VC in range.
-        const I column = (tile * kColumns + lane) * VC;
+        const I column = (tile * lanes + lane) * VC;
+        const I from = VC > 1 && column + VC > w.columns ? w.columns - VC : column;
         const I row_begin = split * w.per_split;
         I row_end = row_begin + w.per_split;
         if (row_end > w.depth) row_end = w.depth;
-        // Contiguous row ranges per group, so group order is index order.
-        const I span = row_end - row_begin;
-        const I per_group = (span + kGroups - 1) / kGroups;
-        I first = row_begin + group * per_group;
-        I last = first + per_group;
-        if (last > row_end) last = row_end;
-        if (first > row_end) first = row_end;
         State s[VC];
 #pragma unroll
         for (int c = 0; c < VC; c++) s[c] = P::init();
-        if (column < w.columns) {
-            const S* base = in + kept_offset(w.outer, outer) + column;
-            I row = first;
-            if (VC == 1) {
-                for (; row + U <= last; row += U) {
+        if (column < w.columns && group < groups) {
+            const S* base = in + kept_offset(w.outer, outer) + from;
+            const I hop = apart ? groups : 1;
+            const I run = apart ? 1 : (row_end - row_begin + groups - 1) / groups;
+            I row = row_begin + group * run;
+            const I end = apart || row + run > row_end ? row_end : row + run;
+            const I next = hop * w.step;
+            const S* at = base + row * w.step;
+            for (; row + (U - 1) * hop < end; row += U * hop, at += U * next) {
+                S v[U][VC];
+#pragma unroll
+                for (int k = 0; k < U; k++) load_columns<NT>(at + k * next, v[k]);
+#pragma unroll
+                for (int c = 0; c < VC; c++) {
                     float x[U];
 #pragma unroll
-                    for (int k = 0; k < U; k++) x[k] = E::widen(base[(row + k) * w.step]);
-                    P::add_chunk(s[0], x, static_cast<uint32_t>(row));
+                    for (int k = 0; k < U; k++) x[k] = E::widen(v[k][c]);
+                    P::template add_packs<U, 1>(s[c], x, static_cast<uint32_t>(row), static_cast<uint32_t>(hop));
                 }
-                for (; row < last; row++) P::add(s[0], E::widen(base[row * w.step]), static_cast<uint32_t>(row));
-            } else {
-                for (; row + U <= last; row += U) {
-                    S v[U][VC];
+            }
+            if (row < end) {
+                const uint32_t left = static_cast<uint32_t>((end - row + hop - 1) / hop);
+                S v[U][VC];
 #pragma unroll
-                    for (int k = 0; k < U; k++) {
-                        const uint4 word = load_word<NT>(base + (row + k) * w.step);
-                        __builtin_memcpy(v[k], &word, 16);
-                    }
+                for (int k = 0; k < U; k++) load_columns<NT>(at + (k < left ? k : 0) * next, v[k]);
 #pragma unroll
-                    for (int c = 0; c < VC; c++) {
-                        float x[U];
+                for (int c = 0; c < VC; c++) {
+                    float x[U];
 #pragma unroll
-                        for (int k = 0; k < U; k++) x[k] = E::widen(v[k][c]);
-                        P::add_chunk(s[c], x, static_cast<uint32_t>(row));
-                    }
-                }
-                for (; row < last; row++) {
-                    S v[VC];
-                    const uint4 word = load_word<NT>(base + row * w.step);
-                    __builtin_memcpy(v, &word, 16);
-#pragma unroll
-                    for (int c = 0; c < VC; c++) P::add(s[c], E::widen(v[c]), static_cast<uint32_t>(row));
+                    for (int k = 0; k < U; k++) x[k] = E::widen(v[k][c]);
+                    P::template add_some<U, 1>(s[c], x, left, static_cast<uint32_t>(row), static_cast<uint32_t>(hop));
                 }
             }
         }
-#pragma unroll
-        for (int c = 0; c < VC; c++) stage[group][c][lane] = s[c];
-        __syncthreads();
+        merge_groups<P, VC>(s, stage, group, groups, lanes);
         if (group == 0 && column < w.columns) {
 #pragma unroll
             for (int c = 0; c < VC; c++) {
-                State t = s[c];
-#pragma unroll
-                for (int g = 1; g < kGroups; g++) t = P::merge(t, stage[g][c][lane]);
-                const I result = outer * w.columns + column + c;
+                if (from + c < column) continue;
+                const I result = outer * w.columns + from + c;
                 if (w.splits == 1) {
-                    Finisher<P>::write(t, f, out, result);
+                    Finisher<P>::write(s[c], f, out, result);
                 } else {
-                    partial[result * w.splits + split] = t;
+                    partial[result * w.splits + split] = s[c];
                 }
             }
         }
-        __syncthreads();
     }
 }
 
@@ -546,6 +673,29 @@ struct Plan {
     uint64_t results, depth;
 };
 
+// The second kernel of a split reduction.
+template <typename P, typename O, typename I>
+int launch_combine(const typename P::State* partial, O* out, uint64_t results, uint64_t splits, const Finish& f,
+                   hipStream_t s, const char* what) {
+    if (splits <= 8) {
+        combine_few_kernel<P, O, I><<<grid_for(results, 256, 64), 256, 0, s>>>(partial, out, static_cast<I>(results),
+                                                                              static_cast<I>(splits), f);
+    } else {
+        combine_kernel<P, O, I><<<grid_for(results, 4, 64), 256, 0, s>>>(partial, out, static_cast<I>(results),
+                                                                        static_cast<I>(splits), f);
+    }
+    return check_launch(what);
+}
+
+// Block states of a split reduction, in a block from the thread's cache.
+template <typename State>
+int split_states(uint64_t count, State** partial) {
+    void* scratch = nullptr;
+    const int status = tc_alloc(count * sizeof(State), &scratch);
+    *partial = static_cast<State*>(scratch);
+    return status;
+}
+
 // The columns kernel over a plan whose innermost kept axis is contiguous and
 // whose one folded axis is strided; VC columns per lane.
 template <typename S, typename P, typename O, int VC, bool NT, typename I>
@@ -556,50 +706,95 @@ int launch_columns(const S* in, O* out, const Plan& plan, const Finish& f, hipSt
     w.outer = make_kept<I>(kept, kept.rank - 1);
     const uint64_t columns = kept.shape[kept.rank - 1];
     const uint64_t outer = results / columns;
-    const uint64_t tiles = (columns + kColumns * VC - 1) / (kColumns * VC);
+    const uint64_t words = (columns + VC - 1) / VC;
+    // Tiles of 64 lanes, or evenly narrower ones where those would leave over
+    // a seventh of the lanes without columns (the constant shape runs a sixth
+    // faster: bf16 [500, 200, 1000] argmax over axis 1, 66 us in tiles of 63
+    // lanes, 56 in 64), the rest of the block on other rows.  Four blocks a CU: what the tiles leave missing is made up by
+    // splitting the depth, each group keeping four rounds of eight rows, since
+    // a split costs a second kernel (2.5 us) and a state a result.
+    const uint64_t want = static_cast<uint64_t>(compute_units()) * 4;
+    uint64_t tiles = (words + 63) / 64;
+    const uint64_t lanes = words * 8 >= tiles * 64 * 7 ? 64 : (words + tiles - 1) / tiles;
+    tiles = (words + lanes - 1) / lanes;
+    const uint64_t groups = std::min<uint64_t>(256 / lanes, depth);
+    const uint64_t base_blocks = outer * tiles;
+    uint64_t splits = 1;
+    if (base_blocks * 2 <= want) {
+        splits = std::min((want + base_blocks - 1) / base_blocks, depth / (groups * 32));
+        if (splits < 2) splits = 1;
+    }
+    const uint64_t per_split = (depth + splits - 1) / splits;
+    splits = (depth + per_split - 1) / per_split;
     w.columns = static_cast<I>(columns);
     w.depth = static_cast<I>(depth);
     w.step = static_cast<I>(plan.folded.strides[0]);
     w.tiles = static_cast<I>(tiles);
     w.tiles_div.set(tiles);
-    // Split the depth across blocks until there are four blocks for every
-    // CU, each row group keeping at least 32 rows (16 of 16-byte words); a
-    // split costs one partial state per result, written and read back once.
-    const uint64_t base_blocks = outer * tiles;
-    const uint64_t want = static_cast<uint64_t>(compute_units()) * 4;
-    uint64_t splits = 1;
-    if (base_blocks < want) {
-        splits = (want + base_blocks - 1) / base_blocks;
-        const uint64_t most = depth / (kGroups * (VC == 1 ? 32 : 16));
-        if (splits > most) splits = most;
-        if (splits < 1) splits = 1;
+    w.splits = static_cast<I>(splits);
+    w.per_split = static_cast<I>(per_split);
+    w.lanes = static_cast<uint32_t>(lanes);
+    w.groups = static_cast<uint32_t>(groups);
+    // Rows of under 64 bytes: neighbouring groups on neighbouring rows share
+    // their lines.  Wider ones: a run of rows a group, since rows a power of
+    // two apart are apt to share a memory channel (f32 [65536 x 2048] sums:
+    // 98 us apart, 82 in runs).
+    w.apart = lanes * VC * sizeof(S) < 64;
+    w.lanes_div = DivMod(w.lanes);
+    const uint64_t blocks = base_blocks * splits;
+    typename P::State* partial = nullptr;
+    int status = splits > 1 ? split_states(splits * results, &partial) : TC_OK;
+    if (status != TC_OK) return status;
+    const uint32_t grid = grid_for(blocks, 1, 64);
+    if (lanes == 64 && groups == 4) {
+        columns_kernel<S, P, O, VC, true, NT, I><<<grid, 256, 0, s>>>(in, out, partial, w, static_cast<I>(blocks), f);
+    } else {
+        columns_kernel<S, P, O, VC, false, NT, I><<<grid, 256, 0, s>>>(in, out, partial, w, static_cast<I>(blocks), f);
     }
-    const uint64_t per_split = (depth + splits - 1) / splits;
+    status = check_launch(what);
+    if (status == TC_OK && splits > 1) status = launch_combine<P, O, I>(partial, out, results, splits, f, s, what);
+    // Stream order keeps the block alive until both kernels have run.
+    if (partial != nullptr) tc_free(partial);
+    return status;
+}
+
+// The rows kernel over a plan whose folded axes are one contiguous run.
+template <typename S, typename P, typename O, bool NT, typename I>
+int launch_rows(const S* in, O* out, const Plan& plan, const Finish& f, hipStream_t s, const char* what) {
+    constexpr uint64_t V = Pack<S>::N;
+    const uint64_t results = plan.results, depth = plan.depth;
+    RowWalk<I> w{};
+    w.kept = make_kept<I>(plan.kept, plan.kept.rank);
+    w.results = static_cast<I>(results);
+    w.depth = static_cast<I>(depth);
+    uint64_t lanes = 64;
+    while (lanes > 1 && depth / V < lanes * 4) lanes /= 2;
+    // A few long slices: cut until there are four waves a CU, each cut eight
+    // rounds of a wave's loads or more.
+    const uint64_t want = static_cast<uint64_t>(compute_units()) * 4, round = 64 * V * 4;
+    uint64_t splits = 1;
+    if (lanes == 64 && results < want) splits = std::min((want + results - 1) / results, depth / (round * 8));
+    if (splits < 2) splits = 1;
+    const uint64_t per_split = splits == 1 ? depth : (depth + splits * V - 1) / (splits * V) * V;
     splits = (depth + per_split - 1) / per_split;
     w.splits = static_cast<I>(splits);
     w.per_split = static_cast<I>(per_split);
-    const uint64_t blocks = base_blocks * splits;
+    w.splits_div.set(splits);
+    w.lanes = static_cast<uint32_t>(lanes);
     typename P::State* partial = nullptr;
-    if (splits > 1) {
-        void* scratch = nullptr;
-        int status = tc_alloc(splits * results * sizeof(typename P::State), &scratch);
-        if (status != TC_OK) return status;
-        partial = static_cast<typename P::State*>(scratch);
+    int status = splits > 1 ? split_states(splits * results, &partial) : TC_OK;
+    if (status != TC_OK) return status;
+    const uint32_t per_block = static_cast<uint32_t>(256 / lanes);
+    const uint32_t blocks = grid_for(results * splits, per_block, 32);
+    if (lanes < 64) {
+        rows_kernel<S, P, O, Rows::few, NT, I><<<blocks, 256, 0, s>>>(in, out, partial, w, f);
+    } else if (splits == 1) {
+        rows_kernel<S, P, O, Rows::whole, NT, I><<<blocks, 256, 0, s>>>(in, out, partial, w, f);
+    } else {
+        rows_kernel<S, P, O, Rows::split, NT, I><<<blocks, 256, 0, s>>>(in, out, partial, w, f);
     }
-    columns_kernel<S, P, O, VC, NT, I><<<grid_for(blocks, 1, 64), 256, 0, s>>>(in, out, partial, w,
-                                                                                 static_cast<I>(blocks), f);
-    int status = check_launch(what);
-    if (status == TC_OK && splits > 1) {
-        if (splits <= 8) {
-            combine_few_kernel<P, O, I><<<grid_for(results, 256, 64), 256, 0, s>>>(
-                partial, out, static_cast<I>(results), static_cast<I>(splits), f);
-        } else {
-            combine_kernel<P, O, I><<<grid_for(results, 4, 64), 256, 0, s>>>(
-                partial, out, static_cast<I>(results), static_cast<I>(splits), f);
-        }
-        status = check_launch(what);
-    }
-    // Stream order keeps the block alive until both kernels have run.
+    status = check_launch(what);
+    if (status == TC_OK && splits > 1) status = launch_combine<P, O, I>(partial, out, results, splits, f, s, what);
     if (partial != nullptr) tc_free(partial);
     return status;
 }
@@ -609,38 +804,26 @@ int launch_reduce(const S* in, O* out, const Plan& plan, const Finish& f, hipStr
     const Axes& kept = plan.kept;
     const Axes& folded = plan.folded;
     const uint64_t results = plan.results, depth = plan.depth;
-    // Rows: the slice is one contiguous run long enough to share a wave.
-    if (folded.rank == 1 && folded.strides[0] == 1 && depth >= 64) {
-        constexpr int V = Pack<S>::N;
-        bool packed = depth % V == 0 && aligned16(in);
-        for (int k = 0; packed && k < kept.rank; k++) packed = (kept.strides[k] * sizeof(S)) % 16 == 0;
-        Kept<I> k = make_kept<I>(kept, kept.rank);
-        const uint32_t blocks = grid_for(results, 4, 32);
-        const bool stream = results * depth * sizeof(S) > kStreamBytes;
-        if (packed && stream) {
-            rows_kernel<S, P, O, true, true, I><<<blocks, 256, 0, s>>>(in, out, k, static_cast<I>(results),
-                                                                       static_cast<I>(depth), f);
-        } else if (packed) {
-            rows_kernel<S, P, O, true, false, I><<<blocks, 256, 0, s>>>(in, out, k, static_cast<I>(results),
-                                                                        static_cast<I>(depth), f);
-        } else {
-            rows_kernel<S, P, O, false, false, I><<<blocks, 256, 0, s>>>(in, out, k, static_cast<I>(results),
-                                                                         static_cast<I>(depth), f);
-        }
-        return check_launch(what);
+    constexpr int VC = 16 / sizeof(S);
+    const bool stream = results * depth * sizeof(S) > kStreamBytes;
+    // Rows: the slice is one contiguous run, of at least a word.
+    if (folded.rank == 1 && folded.strides[0] == 1 && depth >= VC) {
+        if (stream) return launch_rows<S, P, O, true, I>(in, out, plan, f, s, what);
+        return launch_rows<S, P, O, false, I>(in, out, plan, f, s, what);
     }
     // Columns: contiguous neighbouring results, one strided folded axis.
-    if (folded.rank == 1 && kept.rank >= 1 && kept.strides[kept.rank - 1] == 1 &&
-        kept.shape[kept.rank - 1] >= 16) {
-        // An input past the Infinity Cache streams with 16-byte words, VC
-        // columns a lane; a smaller one runs a column a lane, which spreads
-        // it over four times the blocks (measured faster below 256 MiB).
-        constexpr int VC = 16 / sizeof(S);
-        bool packed = results * depth * sizeof(S) > kStreamBytes && kept.shape[kept.rank - 1] % VC == 0 &&
-                      folded.strides[0] % VC == 0 && aligned16(in);
-        for (int k = 0; packed && k + 1 < kept.rank; k++) packed = kept.strides[k] % VC == 0;
-        if (packed) return launch_columns<S, P, O, VC, true, I>(in, out, plan, f, s, what);
-        return launch_columns<S, P, O, 1, false, I>(in, out, plan, f, s, what);
+    if (folded.rank == 1 && kept.rank >= 1 && kept.strides[kept.rank - 1] == 1) {
+        // An input past the Infinity Cache streams with 16-byte words.  A
+        // smaller one takes 4 bytes of columns a lane, which spreads it over
+        // four times the threads, and one column for variances and
+        // arg-reductions, whose arithmetic wants the threads more than the
+        // wider loads (bf16 [150, 77, 513] argmax over axis 1: 8.0 us with
+        // two columns a lane, 7.3 with one).
+        constexpr int kFew = P::kLight ? 4 / sizeof(S) : 1;
+        if (stream && kept.shape[kept.rank - 1] >= static_cast<uint64_t>(VC)) {
+            return launch_columns<S, P, O, VC, true, I>(in, out, plan, f, s, what);
+        }
+        return launch_columns<S, P, O, kFew, false, I>(in, out, plan, f, s, what);
     }
     Kept<I> k = make_kept<I>(kept, kept.rank);
     Folded<I> fo{};
@@ -1002,7 +1185,7 @@ __global__ void __launch_bounds__(256) moments_total_kernel(const S* __restrict_
         const uint64_t packs = n / V;
         for (uint64_t p = first; p < packs; p += stride) {
             float x[V];
-            load_packs<S, 1, false>(reinterpret_cast<const Pack<S>*>(a) + p, x);
+            load_packs<S, 1, false, false, uint64_t>(a, p, 0, 0, x);
             Var::add_chunk(s, x, 0);
         }
         if (blockIdx.x == 0 && threadIdx.x < n - packs * V) Var::add(s, E::widen(a[packs * V + threadIdx.x]), 0);
