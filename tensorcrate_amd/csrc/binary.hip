@@ -335,11 +335,14 @@ struct BinaryWalk {
     Div<I> div[kMaxRank];
     I a[kMaxRank], b[kMaxRank];
     uint32_t step_a, step_b;  // each operand's Step along the run
-    bool vec_a, vec_b;        // a unit-stride operand's groups are 16-byte aligned
 };
 
-// Work items are groups of V consecutive elements of one run (V divides the
-// run).  The output is the row-major layout of the walk's shape.
+// Work items are groups of V consecutive elements of one run, the last of a run
+// possibly shorter.  The output is the row-major layout of the walk's shape.  A
+// whole group moves 16 bytes wherever it starts, so runs that 16 bytes do not
+// divide take words too (bf16 [31, 257, 131] against [1, 257, 1] and
+// [31, 1, 131], us of kernel time: an element a thread 4.5 and 5.4, this 3.9
+// and 4.7; f32 [256, 512, 512], words either way, 110 and 86-88 both).
 template <typename S, typename Op, int V, bool NT, typename I>
 __global__ void __launch_bounds__(256) strided_binary_kernel(const S* __restrict__ a,
                                                              const S* __restrict__ b,
@@ -369,40 +372,37 @@ __global__ void __launch_bounds__(256) strided_binary_kernel(const S* __restrict
             at_a += index * w.a[0];
             at_b += index * w.b[0];
         }
-        float x[V], y[V];
-        if (V > 1 && w.step_a == kUnit && w.vec_a) {
-            Pack<S> p = __builtin_bit_cast(Pack<S>, load_word<NT>(a + at_a + col));
-#pragma unroll
-            for (int k = 0; k < V; k++) x[k] = E::widen(p.v[k]);
-        } else if (w.step_a == kRepeat) {
-            const float v = E::widen(a[at_a]);
-#pragma unroll
-            for (int k = 0; k < V; k++) x[k] = v;
-        } else {
-#pragma unroll
-            for (int k = 0; k < V; k++) x[k] = E::widen(a[at_a + (col + k) * w.a[last]]);
-        }
-        if (V > 1 && w.step_b == kUnit && w.vec_b) {
-            Pack<S> p = __builtin_bit_cast(Pack<S>, load_word<NT>(b + at_b + col));
-#pragma unroll
-            for (int k = 0; k < V; k++) y[k] = E::widen(p.v[k]);
-        } else if (w.step_b == kRepeat) {
-            const float v = E::widen(b[at_b]);
-#pragma unroll
-            for (int k = 0; k < V; k++) y[k] = v;
-        } else {
-#pragma unroll
-            for (int k = 0; k < V; k++) y[k] = E::widen(b[at_b + (col + k) * w.b[last]]);
-        }
         const I o = row * w.shape[last] + col;
-        if (V > 1) {
-            Pack<S> z;
-#pragma unroll
-            for (int k = 0; k < V; k++) z.v[k] = E::narrow(Op::apply(x[k], y[k]));
-            store_word<NT>(out + o, __builtin_bit_cast(uint4, z));
-        } else {
-            out[o] = E::narrow(Op::apply(x[0], y[0]));
+        const I left = w.shape[last] - col;
+        if (V == 1 || left < V) {
+            for (I k = 0; k < V && k < left; k++) {
+                const float x = E::widen(a[at_a + (col + k) * w.a[last]]);
+                const float y = E::widen(b[at_b + (col + k) * w.b[last]]);
+                out[o + k] = E::narrow(Op::apply(x, y));
+            }
+            continue;
         }
+        float x[V], y[V];
+        auto read = [&](float(&v)[V], const S* from, uint32_t step, I apart) {
+            if (step == kUnit) {
+                Pack<S> p = __builtin_bit_cast(Pack<S>, load_any_word<NT>(from + col));
+#pragma unroll
+                for (int k = 0; k < V; k++) v[k] = E::widen(p.v[k]);
+            } else if (step == kRepeat) {
+                const float one = E::widen(*from);
+#pragma unroll
+                for (int k = 0; k < V; k++) v[k] = one;
+            } else {
+#pragma unroll
+                for (int k = 0; k < V; k++) v[k] = E::widen(from[(col + k) * apart]);
+            }
+        };
+        read(x, a + at_a, w.step_a, w.a[last]);
+        read(y, b + at_b, w.step_b, w.b[last]);
+        Pack<S> z;
+#pragma unroll
+        for (int k = 0; k < V; k++) z.v[k % Pack<S>::N] = E::narrow(Op::apply(x[k], y[k]));
+        store_any_word<NT>(out + o, __builtin_bit_cast(uint4, z));
     }
 }
 
@@ -433,35 +433,26 @@ int launch_strided_binary(const S* a, const S* b, S* out, const Walk<3>& walk, u
     auto step_of = [](uint64_t stride) { return stride == 0 ? kRepeat : stride == 1 ? kUnit : kStrided; };
     w.step_a = step_of(walk.strides[0][last]);
     w.step_b = step_of(walk.strides[1][last]);
-    auto runs_aligned = [&](const S* p, int operand) {
-        if (!aligned16(p)) return false;
-        for (int k = 0; k < last; k++) {
-            if ((walk.strides[operand][k] * sizeof(S)) % 16 != 0) return false;
-        }
-        return true;
-    };
-    w.vec_a = runs_aligned(a, 0);
-    w.vec_b = runs_aligned(b, 1);
     const uint64_t run = walk.shape[last];
     constexpr int V = Pack<S>::N;
-    if (run % V == 0 && aligned16(out)) {
-        const uint64_t run_groups = run / V;
-        const uint64_t groups = count / V;
-        Div<I> per_run;
-        per_run.set(run_groups);
+    // Runs shorter than two words, or of elements apart on both sides, take an
+    // element a thread.
+    const bool words = run >= 2 * V && (w.step_a == kUnit || w.step_b == kUnit || run % V == 0);
+    const uint64_t run_groups = words ? (run + V - 1) / V : run;
+    const uint64_t groups = count / run * run_groups;
+    Div<I> per_run;
+    per_run.set(run_groups);
+    const uint32_t blocks = blocks_for(groups, 1);
+    if (!words) {
+        strided_binary_kernel<S, Op, 1, false, I><<<blocks, 256, 0, s>>>(
+            a, b, out, w, static_cast<I>(groups), per_run, static_cast<I>(run_groups));
+    } else if (count * sizeof(S) > kStreamBytes) {
         // Streaming when the output alone exceeds the Infinity Cache.
-        if (count * sizeof(S) > kStreamBytes) {
-            strided_binary_kernel<S, Op, V, true, I><<<blocks_for(groups, 1), 256, 0, s>>>(
-                a, b, out, w, static_cast<I>(groups), per_run, static_cast<I>(run_groups));
-        } else {
-            strided_binary_kernel<S, Op, V, false, I><<<blocks_for(groups, 1), 256, 0, s>>>(
-                a, b, out, w, static_cast<I>(groups), per_run, static_cast<I>(run_groups));
-        }
+        strided_binary_kernel<S, Op, V, true, I><<<blocks, 256, 0, s>>>(
+            a, b, out, w, static_cast<I>(groups), per_run, static_cast<I>(run_groups));
     } else {
-        Div<I> per_run;
-        per_run.set(run);
-        strided_binary_kernel<S, Op, 1, false, I><<<blocks_for(count, 1), 256, 0, s>>>(
-            a, b, out, w, static_cast<I>(count), per_run, static_cast<I>(run));
+        strided_binary_kernel<S, Op, V, false, I><<<blocks, 256, 0, s>>>(
+            a, b, out, w, static_cast<I>(groups), per_run, static_cast<I>(run_groups));
     }
     return check_launch("strided binary");
 }

@@ -308,6 +308,17 @@ __device__ __forceinline__ void store_word(void* p, uint4 v) {
     }
 }
 
+template <bool NT>
+__device__ __forceinline__ void store_any_word(void* p, uint4 v) {
+    u32x4_anywhere* at = static_cast<u32x4_anywhere*>(p);
+    const u32x4 w{v.x, v.y, v.z, v.w};
+    if (NT) {
+        __builtin_nontemporal_store(w, at);
+    } else {
+        *at = w;
+    }
+}
+
 // Blocks of 256 threads for a one-pass kernel over `work` items, `per_thread`
 // items a thread (never zero blocks).  A dispatch holds fewer than 2^32
 // work-items, so past 2^24 - 1 blocks the kernels loop.

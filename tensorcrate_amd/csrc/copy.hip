@@ -6,8 +6,9 @@
 // source/target layout (layout.rs:419-449) and picks one of three kernels:
 //
 //  - rows: both sides step by one along the innermost axis.  Each run is
-//    copied with 16-byte vector accesses when both runs are 16-byte aligned,
-//    which covers contiguous copies, slices and concatenation.
+//    copied with 16-byte accesses wherever it starts, which covers contiguous
+//    copies, slices and concatenation; the pieces of a concatenation go in one
+//    launch.
 //  - tile: one side is contiguous along an axis the other is not (a permute
 //    such as a transpose).  A tile is read along the source's contiguous
 //    axis, held in LDS, and written along the target's, so both HBM streams
@@ -22,6 +23,8 @@
 // of a 288 GB device.
 
 #include <string.h>
+
+#include <algorithm>
 
 #include "common.hpp"
 
@@ -89,45 +92,60 @@ __global__ void __launch_bounds__(256) gather_kernel(const T* __restrict__ src, 
     }
 }
 
-// Rows of `run` words each, a word being one element or 16 bytes of them.
-// `run_div` divides a flat (row, word) index by the words per row.  One word
-// a thread, over a grid that covers them; NT (16-byte words only) marks a
-// copy that streams past the Infinity Cache: its loads are non-temporal, its
-// stores plain (config 3's slice 6.22 -> 6.48 TB/s and concat 6.18 -> 6.50
-// against non-temporal stores).
-template <typename T, bool NT, typename I, int U = 1>
-__global__ void __launch_bounds__(256) rows_kernel(const T* __restrict__ src, T* __restrict__ dst,
-                                                   Layout2<I> layout, Div<I> run_div, I run, I total) {
-    // U words a thread, a grid apart, all loads issued before any store; one
-    // round normally, the loop (64-bit, so it cannot wrap) covering work past
-    // what one dispatch holds.
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; base < total;
-         base += stride * U) {
-        T value[U];
-        I to[U];
-#pragma unroll
-        for (int k = 0; k < U; k++) {
-            const uint64_t item = base + k * stride;
-            if (item < total) {
-                const I i = static_cast<I>(item);
-                I row = run_div.div(i);
-                I word = i - row * run;
-                I from;
-                locate(layout, layout.rank - 1, row, from, to[k]);
-                to[k] += word;
-                if constexpr (NT) {
-                    value[k] = load_word<true>(src + from + word);
-                } else {
-                    value[k] = src[from + word];
-                }
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < U; k++) {
-            if (base + k * stride < total) {
-                dst[to[k]] = value[k];
-            }
+// Rows of `run` elements moved `words` words a row, a word being PER elements
+// (16 bytes, or one element) and a row's last word possibly fewer; `words_div`
+// divides a flat (row, word) index by the words per row.
+template <typename I>
+struct Rows {
+    const void* src;
+    void* dst;
+    Layout2<I> layout;
+    Div<I> words_div;
+    I words, run, total;
+};
+
+// N pieces, each over its own blocks: piece r over blocks first[r] up to
+// first[r + 1].
+template <typename I, int N>
+struct Pieces {
+    Rows<I> piece[N];
+    uint32_t first[N + 1];
+    uint32_t count;
+};
+
+// One word a thread, over a grid that covers them.  Words start anywhere on
+// both sides: runs off 16 bytes (rows of an odd length, slices at an odd place)
+// went an element a thread before (bf16 [31, 128, 131] out of [31, 257, 131]:
+// 2.9 us of kernel time, this 2.5; its two halves joined, 5.9 in two launches,
+// 3.6 in one).  NT (16-byte words only) marks a copy that
+// streams past the Infinity Cache: its loads are non-temporal, its stores plain
+// (config 3's slice 6.22 -> 6.48 TB/s and concat 6.18 -> 6.50 against
+// non-temporal stores).
+template <typename T, int PER, bool NT, typename I, int N>
+__global__ void __launch_bounds__(256) rows_kernel(Pieces<I, N> pieces) {
+    uint32_t r = 0;
+    if constexpr (N > 1) {
+        while (r + 1 < pieces.count && blockIdx.x >= pieces.first[r + 1]) r++;
+    }
+    const Rows<I>& w = pieces.piece[r];
+    const uint32_t block = blockIdx.x - pieces.first[r], blocks = pieces.first[r + 1] - pieces.first[r];
+    // One round normally; the loop (64-bit, so it cannot wrap) covers work
+    // past what one dispatch holds.
+    const uint64_t stride = static_cast<uint64_t>(blocks) * 256;
+    for (uint64_t item = static_cast<uint64_t>(block) * 256 + threadIdx.x; item < w.total; item += stride) {
+        const I i = static_cast<I>(item);
+        const I row = w.words_div.div(i);
+        const I at = (i - row * w.words) * PER;
+        I from, to;
+        locate(w.layout, w.layout.rank - 1, row, from, to);
+        const T* src = static_cast<const T*>(w.src) + from + at;
+        T* dst = static_cast<T*>(w.dst) + to + at;
+        if (PER == 1) {
+            *dst = *src;
+        } else if (at + PER <= w.run) {
+            store_any_word<false>(dst, load_any_word<NT>(src));
+        } else {
+            for (I k = 0; k < w.run - at; k++) dst[k] = src[k];
         }
     }
 }
@@ -176,15 +194,20 @@ __global__ void __launch_bounds__(256) tile_kernel(const T* __restrict__ src, T*
         }
         const I a0 = tile_a * kTile;
         const I b0 = tile_b * kTile;
-        // Read: lanes walk `a`, where the source is contiguous.
-        const I a = a0 + tx;
-        if (a < t.extent_a) {
+        // Read: lanes walk `a`, where the source is contiguous, every row's
+        // load in flight before the first is written to LDS (rows and columns
+        // past the extents repeat the last one).  Loaded where its row was in
+        // range, each row waited for the one before: bf16 [31, 257, 131] with
+        // its last axes exchanged 8.1 us, this 4.1.
+        const I a = a0 + tx < t.extent_a ? a0 + tx : t.extent_a - 1;
+        T v[kTile / kTileRows];
 #pragma unroll
-            for (int r = 0; r < kTile; r += kTileRows) {
-                const I b = b0 + ty + r;
-                if (b < t.extent_b) tile[ty + r][tx] = src[from + a + b * t.src_b];
-            }
+        for (int r = 0; r < kTile; r += kTileRows) {
+            const I b = b0 + ty + r < t.extent_b ? b0 + ty + r : t.extent_b - 1;
+            v[r / kTileRows] = src[from + a + b * t.src_b];
         }
+#pragma unroll
+        for (int r = 0; r < kTile; r += kTileRows) tile[ty + r][tx] = v[r / kTileRows];
         __syncthreads();
         // Write: lanes walk `b`, where the target is contiguous.
         const I b = b0 + tx;
@@ -319,6 +342,42 @@ bool fits32(const Walk<2>& walk, uint64_t count) {
     return true;
 }
 
+// Whether a copy of runs moves them in 16-byte words: runs of at least one.
+template <typename T>
+bool wide_rows(const Walk<2>& walk) {
+    return sizeof(T) < 16 && walk.shape[walk.rank - 1] * sizeof(T) >= 16;
+}
+
+template <typename T, typename I>
+Rows<I> make_rows(const T* src, T* dst, const Walk<2>& walk, uint64_t count) {
+    const uint64_t run = walk.shape[walk.rank - 1];
+    const uint64_t per = wide_rows<T>(walk) ? 16 / sizeof(T) : 1;
+    const uint64_t words = (run + per - 1) / per;
+    Rows<I> w{};
+    w.src = src;
+    w.dst = dst;
+    w.layout = make_layout<I>(walk);
+    w.words_div.set(words);
+    w.words = static_cast<I>(words);
+    w.run = static_cast<I>(run);
+    w.total = static_cast<I>(count / run * words);
+    return w;
+}
+
+template <typename T, typename I, int N>
+int launch_rows(const Pieces<I, N>& pieces, bool stream, bool wide, hipStream_t s) {
+    constexpr int PER = sizeof(T) < 16 ? 16 / sizeof(T) : 1;
+    const uint32_t blocks = pieces.first[pieces.count];
+    if (!wide) {
+        rows_kernel<T, 1, false, I, N><<<blocks, 256, 0, s>>>(pieces);
+    } else if (stream) {
+        rows_kernel<T, PER, true, I, N><<<blocks, 256, 0, s>>>(pieces);
+    } else {
+        rows_kernel<T, PER, false, I, N><<<blocks, 256, 0, s>>>(pieces);
+    }
+    return check_launch("strided copy");
+}
+
 template <typename T, typename I>
 int launch_copy(const T* src, T* dst, const Walk<2>& walk, uint64_t count, bool stream, hipStream_t s) {
     const int rank = walk.rank;
@@ -330,43 +389,11 @@ int launch_copy(const T* src, T* dst, const Walk<2>& walk, uint64_t count, bool 
     const uint64_t inner_src = walk.strides[0][rank - 1];
     const uint64_t inner_dst = walk.strides[1][rank - 1];
     if (inner_src == 1 && inner_dst == 1) {
-        Layout2<I> layout = make_layout<I>(walk);
-        const uint64_t run = walk.shape[rank - 1];
-        const uint64_t rows = count / run;
-        // 16-byte words when every run starts 16-byte aligned.
-        bool wide = sizeof(T) < 16 && (run * sizeof(T)) % 16 == 0 &&
-                    reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
-                    reinterpret_cast<uintptr_t>(dst) % 16 == 0;
-        for (int k = 0; wide && k < rank - 1; k++) {
-            wide = (walk.strides[0][k] * sizeof(T)) % 16 == 0 && (walk.strides[1][k] * sizeof(T)) % 16 == 0;
-        }
-        if (wide) {
-            const uint64_t per = 16 / sizeof(T);
-            Layout2<I> words = layout;
-            for (int k = 0; k < rank - 1; k++) {
-                words.src[k] = static_cast<I>(walk.strides[0][k] / per);
-                words.dst[k] = static_cast<I>(walk.strides[1][k] / per);
-            }
-            const uint64_t run_words = run / per;
-            Div<I> run_div;
-            run_div.set(run_words);
-            const uint64_t total = rows * run_words;
-            if (stream) {
-                rows_kernel<uint4, true, I><<<blocks_for(total, 1), 256, 0, s>>>(
-                    reinterpret_cast<const uint4*>(src), reinterpret_cast<uint4*>(dst), words, run_div,
-                    static_cast<I>(run_words), static_cast<I>(total));
-            } else {
-                rows_kernel<uint4, false, I><<<blocks_for(total, 1), 256, 0, s>>>(
-                    reinterpret_cast<const uint4*>(src), reinterpret_cast<uint4*>(dst), words, run_div,
-                    static_cast<I>(run_words), static_cast<I>(total));
-            }
-        } else {
-            Div<I> run_div;
-            run_div.set(run);
-            rows_kernel<T, false, I><<<blocks_for(count, 1), 256, 0, s>>>(
-                src, dst, layout, run_div, static_cast<I>(run), static_cast<I>(count));
-        }
-        return check_launch("strided copy");
+        Pieces<I, 1> one{};
+        one.piece[0] = make_rows<T, I>(src, dst, walk, count);
+        one.first[1] = blocks_for(one.piece[0].total, 1);
+        one.count = 1;
+        return launch_rows<T, I, 1>(one, stream, wide_rows<T>(walk), s);
     }
     // A permute: find the axis the source is contiguous along and the one
     // the target is, distinct and both long enough to fill a tile.
@@ -479,6 +506,92 @@ int copy_by_width(uint32_t width, const void* src, void* dst, const Walk<2>& wal
     }
 }
 
+// ---- the pieces of an assemble in one launch -----------------------------------
+
+constexpr uint32_t kPieces = 8;
+
+// A region's box in the row-major grid its target strides step through: the
+// first coordinate along each axis.  False where the strides are no such grid
+// or the box does not stay inside a row of it.
+bool box_of(const tc_region& region, uint64_t (&first)[kMaxRank]) {
+    uint64_t left = region.to.offset;
+    for (uint32_t k = 0; k < region.rank; k++) {
+        const uint64_t step = region.to.strides[k];
+        if (step == 0 || (k > 0 && region.to.strides[k - 1] % step != 0)) return false;
+        first[k] = left / step;
+        left %= step;
+        if (k > 0 && first[k] + region.shape[k] > region.to.strides[k - 1] / step) return false;
+    }
+    return left == 0;
+}
+
+// Whether two regions are boxes of one grid with no element in common.
+bool apart(const tc_region& a, const tc_region& b) {
+    if (a.rank != b.rank) return false;
+    uint64_t fa[kMaxRank], fb[kMaxRank];
+    if (!box_of(a, fa) || !box_of(b, fb)) return false;
+    bool disjoint = false;
+    for (uint32_t k = 0; k < a.rank; k++) {
+        if (a.to.strides[k] != b.to.strides[k]) return false;
+        disjoint |= fa[k] + a.shape[k] <= fb[k] || fb[k] + b.shape[k] <= fa[k];
+    }
+    return disjoint;
+}
+
+// Checked regions copied in their order into `dst`, of `len` T's: neighbouring
+// ones that are contiguous runs on both sides, share no target element and
+// read nothing of the target go in one launch, up to kPieces of them (a launch
+// costs 2-3 us where a piece is small); the rest one by one, through `other`.
+template <typename T, class Other>
+int assemble_pieces(void* dst, uint64_t len, const tc_region* regions, uint32_t count, bool stream, hipStream_t s,
+                    const Other& other) {
+    Pieces<uint32_t, kPieces> pieces{};
+    uint32_t held[kPieces];
+    auto flush = [&]() {
+        int status = TC_OK;
+        if (pieces.count == 1) {
+            status = other(regions[held[0]]);
+        } else if (pieces.count > 1) {
+            status = launch_rows<T, uint32_t, static_cast<int>(kPieces)>(pieces, stream, true, s);
+        }
+        pieces.count = 0;
+        return status;
+    };
+    const uintptr_t begin = reinterpret_cast<uintptr_t>(dst), end = begin + len * sizeof(T);
+    for (uint32_t r = 0; r < count; r++) {
+        const tc_region& region = regions[r];
+        uint64_t elements = 1;
+        for (uint32_t k = 0; k < region.rank; k++) elements *= region.shape[k];
+        if (elements == 0) continue;
+        const uint64_t* strides[2] = {region.from.strides, region.to.strides};
+        const uint64_t offsets[2] = {region.from.offset, region.to.offset};
+        const Walk<2> walk = coalesce<2>(region.rank, region.shape, strides, offsets);
+        const uintptr_t source = reinterpret_cast<uintptr_t>(region.source);
+        const bool joins = walk.rank > 0 && walk.strides[0][walk.rank - 1] == 1 &&
+                           walk.strides[1][walk.rank - 1] == 1 && wide_rows<T>(walk) && fits32(walk, elements) &&
+                           (source >= end || source + region.source_len * sizeof(T) <= begin);
+        bool fits = joins && pieces.count < kPieces;
+        for (uint32_t h = 0; fits && h < pieces.count; h++) fits = apart(regions[held[h]], region);
+        if (!fits) {
+            const int status = flush();
+            if (status != TC_OK) return status;
+        }
+        if (!joins) {
+            const int status = other(region);
+            if (status != TC_OK) return status;
+            continue;
+        }
+        const uint32_t at = pieces.count++;
+        held[at] = r;
+        pieces.piece[at] = make_rows<T, uint32_t>(static_cast<const T*>(region.source) + walk.offsets[0],
+                                                  static_cast<T*>(dst) + walk.offsets[1], walk, elements);
+        // A piece's share of what one dispatch holds.
+        pieces.first[at + 1] =
+            pieces.first[at] + std::min<uint32_t>(blocks_for(pieces.piece[at].total, 1), 0xffffffu / kPieces);
+    }
+    return flush();
+}
+
 // One region: `shape` from `source` at `from` to `target` at `to`, as part
 // of an operation moving `traffic` bytes (0: just this region).
 int write_region(uint32_t width, const void* source, uint64_t source_len, void* target,
@@ -544,10 +657,21 @@ int tc_assemble(uint32_t width, void* dst, uint64_t len, const tc_region* region
         if (elements != 0 && any_null({region.source, dst})) return null_operand("assemble");
         traffic += 2 * elements * width;
     }
+    auto one = [&](const tc_region& region) {
+        return write_region(width, region.source, region.source_len, dst, len, region.rank, region.shape, region.from,
+                            region.to, traffic, "assemble");
+    };
+    TC_STREAM(s);
+    const bool stream = traffic >= kStreamBytes;
+    switch (width) {
+        case 1: return assemble_pieces<Word<1>::type>(dst, len, regions, count, stream, s, one);
+        case 2: return assemble_pieces<Word<2>::type>(dst, len, regions, count, stream, s, one);
+        case 4: return assemble_pieces<Word<4>::type>(dst, len, regions, count, stream, s, one);
+        case 8: return assemble_pieces<Word<8>::type>(dst, len, regions, count, stream, s, one);
+        default: break;
+    }
     for (uint32_t r = 0; r < count; r++) {
-        const tc_region& region = regions[r];
-        int status = write_region(width, region.source, region.source_len, dst, len, region.rank,
-                                  region.shape, region.from, region.to, traffic, "assemble");
+        const int status = one(regions[r]);
         if (status != TC_OK) return status;
     }
     return TC_OK;
