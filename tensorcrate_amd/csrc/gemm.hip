@@ -22,12 +22,7 @@
 // fragments are read under that slice's matrix-core steps.
 //
 // f32 operands (v_mfma_f32_16x16x4_f32, the in-place f32 kernel) are read in
-// place the same way, a row-contiguous operand's four k per lane coming from
-// four LDS reads down its tile; 256 x 128 tiles (128 x 128 for products with
-// fewer such tiles than CUs), 32-deep steps.  One 16-byte
-// LDS read of a K-contiguous f32 tile feeds four consecutive matrix-core
-// steps, since the sum over k does not care which lane holds which k as long
-// as both operands agree.
+// place the same way, in 128 x 128 or 128 x 64 tiles and 32-deep steps.
 //
 // Products too small to give those tiles to most CUs, and operands whose rows
 // are not 16-byte aligned, take the register-fed kernel (gemm_sliced.hpp).
@@ -48,6 +43,7 @@
 
 #include "common.hpp"
 #include "gemm_kernels.hpp"
+#include "gemm_rules.hpp"
 #include "gemm_sliced.hpp"
 #include "program.hpp"
 
@@ -343,23 +339,13 @@ void launch_tiled16(const S* a, const S* b, O* c, uint32_t m, uint32_t k, uint32
     }
 }
 
-// The in-place f32 kernel's shape: 128 x 128 tiles over four waves of 64 x
-// 64, whatever the product's size.  At 70 KiB of LDS and 82 VGPRs + 64 AGPRs
-// two blocks share a CU, so one block's step barrier and first fragment
-// reads overlap the other's matrix-core steps; 256 x 128 tiles (one block a
-// CU) measured 4-16% slower on every shape tried on MI355X, from 2048^3 to
-// 8192^3 in all three forms (4096^3: 132.2 / 133.6 / 129.4 TFLOP/s PLAIN /
-// LEFT / RIGHT against 124.9 / 118.7 / 124.5), with the same bits.
+// The in-place f32 kernel, in 128 x 128 or 128 x 64 tiles (`narrow32`).
 template <typename O, bool A_KC, bool B_KC, class EPI = PlainStore>
 void launch_inplace32(const float* a, const float* b, O* c, uint32_t m, uint32_t k, uint32_t n, bool accumulate,
                       hipStream_t s, const EPI& epi = EPI{}) {
-    const uint32_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
-    // Too few 128 x 128 tiles for two blocks on every CU (a 4096 x 1024
-    // product has 256): 128 x 64 tiles, twice the blocks, so the two-blocks-
-    // a-CU overlap still happens.
+    const uint32_t tiles = ((m + 127) / 128) * ((n + 127) / 128), narrow = ((m + 127) / 128) * ((n + 63) / 64);
     if constexpr (!EPI::kProgram) {
-        if (tiles < 2 * static_cast<uint32_t>(compute_units())) {
-            const uint32_t narrow = ((m + 127) / 128) * ((n + 63) / 64);
+        if (narrow32(m, n)) {
             inplace32_kernel<O, A_KC, B_KC, 128, 64, EPI><<<narrow, kThreads, 0, s>>>(a, b, c, m, n, k, accumulate,
                                                                                      epi);
             return;
@@ -368,43 +354,7 @@ void launch_inplace32(const float* a, const float* b, O* c, uint32_t m, uint32_t
     inplace32_kernel<O, A_KC, B_KC, 128, 128, EPI><<<tiles, kThreads, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
 }
 
-// ---- register-fed products -----------------------------------------------------------
-//
-// The sliced kernel's tile for a product: 64 x 64 where that gives at least
-// half the CUs a block, else 32 x 32 where that does, else 16 x 16, and never
-// a tile twice the product's smaller side.  More, smaller tiles fill the chip
-// but read the operands more often (us a call): f32 768^3, 144 / 576 tiles of
-// 64 / 32: 17.7 / 20.0; f32 512^3, 64 / 256: 12.6 / 5.8; f32 256 x 8192 x 256,
-// 64 / 256 tiles of 32 / 16: 44 / 27; bf16 64 x 4096 x 4096 with B transposed,
-// 64 / 256 / 1024 of 64 / 32 / 16: 32 / 17 / 45.
-uint32_t sliced_tile(uint32_t m, uint32_t n) {
-    const uint64_t cus = static_cast<uint64_t>(compute_units());
-    const uint32_t narrow = std::min(m, n);
-    for (uint32_t tile = 64; tile > 16; tile /= 2) {
-        const uint64_t blocks = static_cast<uint64_t>((m + tile - 1) / tile) * ((n + tile - 1) / tile);
-        if (narrow > tile / 2 && blocks * 2 >= cus) return tile;
-    }
-    return 16;
-}
-
-// Whether a product whose operands the tiled kernels can read is small enough
-// for the sliced kernel instead.  A tiled 16-bit block does a 64-deep step in
-// about 0.8 us whether or not the other CUs have a tile, while the sliced
-// kernel runs at 300-320 TFLOP/s on these: they meet near half a 128 x 128
-// tile a CU (us a call, tiled / sliced: 64 tiles, 1024^3, 14.8 / 9.3; 192,
-// 2048 x 1024 x 1536, 15.5 / 21.8).  f32's matrix cores are sixteen times
-// slower, so the sliced kernel's extra reads hide for longer: 64 tiles
-// 44.9 / 22.4, 192 tiles 71.7 / 73.
-bool small_product(uint32_t m, uint32_t n, bool f32) {
-    const uint64_t tiles = static_cast<uint64_t>((m + 127) / 128) * ((n + 127) / 128);
-    return tiles * 4 < static_cast<uint64_t>(compute_units()) * (f32 ? 3 : 2);
-}
-
-// The sliced kernel addresses its operands with 32-bit byte offsets.
-bool sliced_reach(uint64_t m, uint64_t k, uint64_t n, size_t width) {
-    const uint64_t limit = uint64_t{1} << 31;
-    return m * k * width < limit && k * n * width < limit;
-}
+// ---- register-fed products (gemm_rules.hpp says which) ---------------------------------
 
 template <typename S, typename O, bool A_KC, bool B_KC, class EPI = PlainStore>
 void launch_sliced(const S* a, const S* b, O* c, uint32_t m, uint32_t k, uint32_t n, bool accumulate, hipStream_t s,

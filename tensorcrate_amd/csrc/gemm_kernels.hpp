@@ -132,6 +132,24 @@ struct PlainStore {
     static constexpr bool kProgram = false;
 };
 
+// Plain stores of a product whose operands were copied to rows of whole 16-byte
+// words, zeros after their own elements: the rows' lengths, in elements, where
+// they are not the product's extents.
+struct PaddedStore {
+    static constexpr bool kProgram = false;
+    uint32_t lda, ldb;
+};
+template <class EPI>
+__device__ __forceinline__ uint32_t row_a(const EPI& epi, uint32_t own) {
+    if constexpr (std::is_same<EPI, PaddedStore>::value) return epi.lda;
+    return own;
+}
+template <class EPI>
+__device__ __forceinline__ uint32_t row_b(const EPI& epi, uint32_t own) {
+    if constexpr (std::is_same<EPI, PaddedStore>::value) return epi.ldb;
+    return own;
+}
+
 // Whether an epilogue type also has the run form (`kRuns`, with
 // `Invariant`, `invariant` and `run`); a type without the member has not.
 template <class EPI, class = void>
@@ -220,15 +238,15 @@ __device__ __forceinline__ void program_pass(const EPI& epi, float* r0, float* r
 // consecutive runs, each thread on the same four columns in every round
 // (BN / 4 divides the workgroup), whose row-invariant loads `inv` holds.
 template <int BN, int G, int REGION_ROWS, int H, int WAVE_ROWS, class EPI>
-__device__ __forceinline__ void program_runs(const EPI& epi, const typename EPI::Invariant& inv, float* region,
-                                             uint32_t rows, uint32_t pass, uint32_t row_base, uint32_t col_base,
-                                             uint32_t M, uint32_t N) {
+__device__ __forceinline__ void program_runs(const EPI& epi, const typename EPI::Invariant& inv, float* r0, float* r1,
+                                             float* r2, float* r3, uint32_t rows, uint32_t pass, uint32_t row_base,
+                                             uint32_t col_base, uint32_t M, uint32_t N) {
     constexpr uint32_t kPerRow = BN / 4;
     const uint32_t runs = rows * kPerRow;
     for (uint32_t q = threadIdx.x; q < runs; q += blockDim.x) {
         const uint32_t rr = q / kPerRow, cc = (q % kPerRow) * 4;
         const float4 v =
-            *reinterpret_cast<const float4*>(staged_at<BN, G, REGION_ROWS>(region, region, region, region, rr, cc));
+            *reinterpret_cast<const float4*>(staged_at<BN, G, REGION_ROWS>(r0, r1, r2, r3, rr, cc));
         const float product[4] = {v.x, v.y, v.z, v.w};
         const uint32_t row = row_base + (rr / H) * WAVE_ROWS + pass * H + rr % H;
         const uint32_t col = col_base + cc;
@@ -238,202 +256,6 @@ __device__ __forceinline__ void program_runs(const EPI& epi, const typename EPI:
 
 constexpr int kBK32 = 32;
 constexpr int kLd32 = kBK32 + 4;
-
-// ---- f32 operands in place ---------------------------------------------------------
-//
-// The f32 product with each operand read in its stored orientation, as the
-// 16-bit kernel does, so `matmul_transposed_add` (the tape's backward
-// products) and a plain `matmul` pay for no transpose pass.  A lane's four k
-// for one tile row come from one ds_read_b128 of a K-contiguous tile, or
-// four ds_read_b32 down a row-contiguous tile ([k][rows + 4]: the 4-float
-// pad puts the four k-rows a wave reads on distinct bank quarters).  A
-// K-contiguous tile's rows are 128 bytes, 16-byte chunk c of row r at
-// c ^ ((r / 2) % 8): conflict-free for the 16 rows a ds_read_b128 reads,
-// where rows padded to 144 bytes measured a 2-way conflict on every read
-// (16.8M conflict cycles a 4096^3 launch for each such operand).  HBM is
-// staged through buffer loads (zeros past the operand) into registers and
-// then LDS, double-buffered, 256 x 128 or 128 x 128 tiles, 32-deep steps,
-// four waves of a quarter tile.  Requirements as for the 16-bit kernel, with K (K-contiguous)
-// or the contiguous extent (row-contiguous) a multiple of 4.
-
-template <int ROWS, bool KC>
-struct Stager32 {
-    static constexpr int kRowChunks = KC ? kBK32 / 4 : ROWS / 4;  // 16-byte chunks per tile row
-    static constexpr int kPassRows = kThreads / kRowChunks;
-    static constexpr int kPasses = (KC ? ROWS : kBK32) / kPassRows;
-    static constexpr int kLdsRow = KC ? kBK32 : ROWS + 4;
-    static constexpr int kTile = KC ? ROWS * kLdsRow : kBK32 * kLdsRow;  // floats a stage
-    static_assert(!KC || kPassRows % 16 == 0, "a pass's rows repeat the swizzle");
-    __device__ static __forceinline__ int swizzle(int row) { return (row / 2) % 8; }
-    __amdgpu_buffer_rsrc_t rsrc;
-    uint32_t offset, pass_bytes, k_bytes, lds_at, k_in;
-
-    __device__ void init(const float* p, uint32_t first, uint32_t rows, uint32_t ld, uint32_t depth, int t) {
-        const uint32_t row = t / kRowChunks, part = (t % kRowChunks) * 4;
-        if (KC) {
-            rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p + static_cast<uint64_t>(first) * ld), 0,
-                                                     (rows - first) * ld * 4, kBufferFlags);
-            k_bytes = 4;
-            k_in = part;
-        } else {
-            rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p + first), 0, (depth * ld - first) * 4,
-                                                     kBufferFlags);
-            k_bytes = ld * 4;
-            k_in = 0;
-        }
-        offset = (row * ld + part) * 4;
-        pass_bytes = kPassRows * ld * 4;
-        lds_at = row * kLdsRow + (KC ? ((part / 4) ^ swizzle(row)) * 4 : part);
-    }
-    __device__ __forceinline__ void fetch(uint4 (&stage)[kPasses], uint32_t k0, uint32_t K, bool full) const {
-        const uint32_t at = (full || !KC || k0 + k_in < K) ? offset : 0x80000000u;
-#pragma unroll
-        for (int i = 0; i < kPasses; i++) {
-            auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, i * pass_bytes + k0 * k_bytes, 0);
-            stage[i] = __builtin_bit_cast(uint4, v);
-        }
-    }
-    __device__ __forceinline__ void commit(const uint4 (&stage)[kPasses], float* lds) const {
-        uint4* to = reinterpret_cast<uint4*>(lds);
-#pragma unroll
-        for (int i = 0; i < kPasses; i++) to[(lds_at + i * kPassRows * kLdsRow) / 4] = stage[i];
-    }
-    // Lane `lane`'s four k (4 (lane / 16) + 0..3 of the slice at `kk`) of
-    // tile row `row`.
-    __device__ __forceinline__ f32x4 fragment(const float* lds, int row, int kk, int lane) const {
-        const int k = kk + (lane / 16) * 4;
-        if (KC) return reinterpret_cast<const f32x4*>(lds)[row * (kLdsRow / 4) + ((k / 4) ^ swizzle(row))];
-        return f32x4{lds[k * kLdsRow + row], lds[(k + 1) * kLdsRow + row], lds[(k + 2) * kLdsRow + row],
-                     lds[(k + 3) * kLdsRow + row]};
-    }
-};
-
-// BM x BN tiles over four waves of (BM / 2) x (BN / 2).
-template <typename O, bool A_KC, bool B_KC, int BM, int BN, class EPI = PlainStore>
-__global__ void __launch_bounds__(kThreads) inplace32_kernel(const float* __restrict__ A, const float* __restrict__ B,
-                                                             O* __restrict__ C, uint32_t M, uint32_t N, uint32_t K,
-                                                             bool accumulate, EPI epi) {
-    using SA = Stager32<BM, A_KC>;
-    using SB = Stager32<BN, B_KC>;
-    constexpr int TM = BM / 32, TN = BN / 32;  // 16 x 16 tiles per wave
-    constexpr int kA = SA::kTile;
-    constexpr int kB = SB::kTile;
-    __shared__ __attribute__((aligned(16))) float lds_a[2 * kA];
-    __shared__ __attribute__((aligned(16))) float lds_b[2 * kB];
-    const uint32_t tiles_m = (M + BM - 1) / BM;
-    const uint32_t tiles_n = (N + BN - 1) / BN;
-    uint32_t tm, tn;
-    tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    const uint32_t m0 = tm * BM, n0 = tn * BN;
-    const int t = threadIdx.x;
-    const int lane = t % 64;
-    const int wave = t / 64;
-    const int wm = wave / 2, wn = wave % 2;
-    SA sa;
-    SB sb;
-    sa.init(A, m0, M, A_KC ? K : M, K, t);
-    sb.init(B, n0, N, B_KC ? K : N, K, t);
-    uint4 stage_a[SA::kPasses], stage_b[SB::kPasses];
-
-    f32x4 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = f32x4{};
-
-    const uint32_t steps = (K + kBK32 - 1) / kBK32;
-    if (steps > 0) {
-        sa.fetch(stage_a, 0, K, kBK32 <= K);
-        sb.fetch(stage_b, 0, K, kBK32 <= K);
-        sa.commit(stage_a, lds_a);
-        sb.commit(stage_b, lds_b);
-        __syncthreads();
-    }
-    const int row_in = lane % 16;
-    for (uint32_t step = 0; step < steps; step++) {
-        const int buffer = step & 1;
-        const bool more = step + 1 < steps;
-        if (more) {
-            const uint32_t k0 = (step + 1) * kBK32;
-            sa.fetch(stage_a, k0, K, k0 + kBK32 <= K);
-            sb.fetch(stage_b, k0, K, k0 + kBK32 <= K);
-        }
-        const float* la = lds_a + buffer * kA;
-        const float* lb = lds_b + buffer * kB;
-#pragma unroll
-        for (int kk = 0; kk < kBK32; kk += 16) {
-            f32x4 a[TM], b[TN];
-#pragma unroll
-            for (int i = 0; i < TM; i++) a[i] = sa.fragment(la, wm * (BM / 2) + i * 16 + row_in, kk, lane);
-#pragma unroll
-            for (int j = 0; j < TN; j++) b[j] = sb.fragment(lb, wn * (BN / 2) + j * 16 + row_in, kk, lane);
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int i = 0; i < TM; i++)
-#pragma unroll
-                    for (int j = 0; j < TN; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
-        }
-        if (more) {
-            sa.commit(stage_a, lds_a + (buffer ^ 1) * kA);
-            sb.commit(stage_b, lds_b + (buffer ^ 1) * kB);
-        }
-        __syncthreads();
-    }
-
-    if constexpr (EPI::kProgram) {
-        // Passes of a power-of-two number of rows that fit in both A stages,
-        // each taking the same share of both wave rows.
-        constexpr int kFit = 2 * kA / BN;
-        constexpr int kPass = kFit >= 128 ? 128 : 64;
-        constexpr int kPasses = BM / kPass, H = BM / 2 / kPasses;
-        static_assert(kFit >= kPass && BM % kPass == 0 && H % 16 == 0, "a pass fits in LDS");
-        // The run form loads what every row reads alike for the thread's
-        // four columns before any store, so no load waits behind one.
-        typename RunState<EPI>::Invariant inv{};
-        if constexpr (HasRuns<EPI>::value) {
-            static_assert(kThreads % (BN / 4) == 0, "a thread keeps its columns in every round");
-            const uint32_t col = n0 + (threadIdx.x % (BN / 4)) * 4;
-            epi.invariant(inv, col < N, col);
-        }
-#pragma unroll
-        for (int pass = 0; pass < kPasses; pass++) {
-            lds_barrier();  // every wave is done with LDS
-#pragma unroll
-            for (int i = pass * H / 16; i < (pass + 1) * H / 16; i++) {
-#pragma unroll
-                for (int j = 0; j < TN; j++) {
-                    const uint32_t col = wn * (BN / 2) + j * 16 + lane % 16;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const uint32_t rr = wm * H + i * 16 - pass * H + 4 * (lane / 16) + e;
-                        *staged_at<BN, 16, kPass>(lds_a, lds_a, lds_a, lds_a, rr, col) = acc[i][j][e];
-                    }
-                }
-            }
-            lds_barrier();
-            if constexpr (HasRuns<EPI>::value) {
-                program_runs<BN, 16, kPass, H, BM / 2>(epi, inv, lds_a, kPass, pass, m0, n0, M, N);
-            } else {
-                program_pass<BN, 16, kPass, H, BM / 2>(epi, lds_a, lds_a, lds_a, lds_a, kPass, pass, m0, n0, M, N);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const uint32_t col = n0 + wn * (BN / 2) + j * 16 + lane % 16;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const uint32_t row = m0 + wm * (BM / 2) + i * 16 + 4 * (lane / 16) + e;
-                    if (row < M && col < N) store_out(C, static_cast<uint64_t>(row) * N + col, acc[i][j][e], accumulate);
-                }
-            }
-        }
-    }
-}
 
 // ---- 16-bit operands in place ---------------------------------------------------------
 //
@@ -639,8 +461,8 @@ __global__ void __launch_bounds__(WM * WN * 64) direct16_kernel(const S* __restr
     using StagerB = DirectStager<S, BN, B_KC, kWaves, BK>;
     StagerA sa;
     StagerB sb;
-    sa.init(A, m0, M, A_KC ? K : M, K, wave, lane);
-    sb.init(B, n0, N, B_KC ? K : N, K, wave, lane);
+    sa.init(A, m0, M, row_a(epi, A_KC ? K : M), K, wave, lane);
+    sb.init(B, n0, N, row_b(epi, B_KC ? K : N), K, wave, lane);
 
     f32x16 acc[TM][TN];
 #pragma unroll
@@ -988,6 +810,246 @@ __device__ __forceinline__ void store_quad(O* at, f32x4 v, bool accumulate) {
     }
 }
 
+// ---- f32 operands in place ---------------------------------------------------------
+//
+// The f32 product with each operand read in its stored orientation, as the
+// 16-bit kernels do, so `matmul_transposed_add` (the tape's backward products)
+// and a plain `matmul` pay for no transpose pass: 128 x BN tiles over four waves
+// of 64 x BN / 2, 16 x 16 x 4 matrix-core steps, 32-deep K steps in two LDS
+// stages filled by direct loads.
+//  - A K-contiguous stage tile is 128-byte rows, 16-byte chunk c of row r at
+//    c ^ ((r / 2) % 8); a lane's four k of one row come from one ds_read_b128 and
+//    feed four consecutive matrix-core steps, since the sum over k does not care
+//    which lane holds which k as long as both operands agree.
+//  - A row-contiguous tile is rows of one k.  A lane reads its 4 (BN = 64: B's 2)
+//    consecutive rows of one k at once: fragment i of a wave is then rows
+//    4 x + i, x = 0 .. 15, rather than 16 i + x, which only the stores have to
+//    know.  Reading rows 16 i + x took four ds_read_b32 a fragment.
+//  - Step s computes its first 16-deep slice from registers while the second's
+//    fragments are read; after the barrier that follows, its stage is free for
+//    step s + 2's direct loads, and the second slice runs while step s + 1's
+//    first fragments are read.  So no slice waits for its own LDS reads, which
+//    matters where a CU has one block (a 4096 x 1024 product has 256 tiles of 128
+//    x 128): the kernel before this one, staged through registers with its reads
+//    at each slice's start, kept the matrix cores 74% busy on 128 x 64 tiles there
+//    and 86% with two blocks a CU.
+//  - Operands are swapped into the matrix-core step (B's fragment first), so a
+//    lane holds runs of consecutive columns of C.
+// us a call (PLAIN / LEFT / RIGHT) with that kernel and with this: 4096^3 1014 /
+// 1024 / 1039 and 913 / 902 / 909 (150-152 TFLOP/s; these matrix-core steps alone
+// reach 154); 4096 x 1024 x 4096 264 / 266 / 270 and 239 / 235 / 235; 4096 x 4096 x
+// 1024 272 / 288 / 290 and 237 / 234 / 233; 2048^3 139 / 147 / 147 and 125 / 121 /
+// 120.
+// Requirements: operands 16-byte aligned row by row and under 2^31 bytes.
+
+template <int ROWS, bool KC>
+struct Stager32 {
+    static constexpr int kPer = ROWS / 8 / 4;  // 1 KiB instructions a wave
+    static constexpr int kLanesPerRow = KC ? 8 : ROWS / 4;
+    static constexpr int kRowsPer = 64 / kLanesPerRow;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t offset, k_of, stride, k_bytes;
+    int wave;
+
+    __device__ void init(const float* p, uint32_t first, uint32_t rows, uint32_t ld, uint32_t depth, int w, int lane) {
+        wave = w;
+        const uint32_t row = kRowsPer * w + lane / kLanesPerRow;
+        const uint32_t chunk = (lane % kLanesPerRow) ^ (KC ? (row / 2) % 8 : 0);
+        if (KC) {
+            rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p + static_cast<uint64_t>(first) * ld), 0,
+                                                     (rows - first) * ld * 4, kBufferFlags);
+        } else {
+            rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p + first), 0, (depth * ld - first) * 4,
+                                                     kBufferFlags);
+        }
+        k_bytes = KC ? 4 : ld * 4;
+        k_of = KC ? chunk * 4 : 0;
+        offset = (row * ld + chunk * 4) * 4;
+        // From one of a wave's instructions to its next: a whole number of the
+        // swizzle's 16 rows (KC: 32).
+        stride = kRowsPer * 4 * ld * 4;
+    }
+    // Past K a K-contiguous chunk is the next row's, so it is pointed past the
+    // resource (operands are under 2^31 bytes) and loads zeros.
+    __device__ __forceinline__ void fetch(float* tile, uint32_t k0, uint32_t K, bool full) const {
+        const uint32_t at = (full || !KC || k0 + k_of < K) ? offset : 0x80000000u;
+#pragma unroll
+        for (int i = 0; i < kPer; i++) {
+            uint8_t* dst = reinterpret_cast<uint8_t*>(tile) + 1024 * (wave + 4 * i);
+            const uint32_t soffset = __builtin_amdgcn_readfirstlane(k0 * k_bytes + i * stride);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)dst, 16, at,
+                                                     soffset, 0, 0);
+        }
+    }
+};
+
+// A wave's T fragments of the 16-deep slice `q` of a stage tile of ROWS rows,
+// from tile row `first` on: f[i][e] is k 16 q + 4 (lane / 16) + e.
+template <int ROWS, bool KC, int T>
+__device__ __forceinline__ void read32(float (&f)[T][4], const float* tile, int first, int q, int lane) {
+    const int x = lane % 16, g = lane / 16;
+    if constexpr (KC) {
+        const int r = first + x;
+        const uint8_t* at = reinterpret_cast<const uint8_t*>(tile) + r * 128 + (((4 * q + g) ^ ((r / 2) % 8)) * 16);
+#pragma unroll
+        for (int i = 0; i < T; i++) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(at + 2048 * i);
+#pragma unroll
+            for (int e = 0; e < 4; e++) f[i][e] = v[e];
+        }
+    } else {
+        typedef float run __attribute__((ext_vector_type(T)));
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const run v = *reinterpret_cast<const run*>(tile + (16 * q + 4 * g + e) * ROWS + first + T * x);
+#pragma unroll
+            for (int i = 0; i < T; i++) f[i][e] = v[i];
+        }
+    }
+}
+
+template <typename O, bool A_KC, bool B_KC, int BM, int BN, class EPI = PlainStore>
+__global__ void __launch_bounds__(kThreads) inplace32_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                             O* __restrict__ C, uint32_t M, uint32_t N, uint32_t K,
+                                                             bool accumulate, EPI epi) {
+    static_assert(BM == 128 && (BN == 128 || BN == 64), "four waves of 64 x BN / 2");
+    constexpr int TM = 4, TN = BN / 32;
+    constexpr int kA = BM * kBK32, kB = BN * kBK32;
+    using StagerA = Stager32<BM, A_KC>;
+    using StagerB = Stager32<BN, B_KC>;
+    constexpr int kLoads = StagerA::kPer + StagerB::kPer;
+    constexpr int kReads = 4 + (B_KC ? TN : 4);
+    constexpr int kSteps = 4 * TM * TN;  // matrix-core steps of a slice
+    uint32_t tm, tn;
+    tile_of(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN, tm, tn);
+    const uint32_t m0 = tm * BM, n0 = tn * BN;
+    const int lane = threadIdx.x % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int wm = wave / 2, wn = wave % 2;
+    StagerA sa;
+    StagerB sb;
+    sa.init(A, m0, M, row_a(epi, A_KC ? K : M), K, wave, lane);
+    sb.init(B, n0, N, row_b(epi, B_KC ? K : N), K, wave, lane);
+
+    const uint32_t steps = (K + kBK32 - 1) / kBK32;
+    // Step s; past the last step, a harmless reload of it.
+    auto stage_of = [&](auto t, uint32_t s) __attribute__((always_inline)) {
+        const uint32_t k0 = (s < steps ? s : steps - 1) * kBK32;
+        sa.fetch(stage_tile<float, kA, 2 * decltype(t)::value>(), k0, K, k0 + kBK32 <= K);
+        sb.fetch(stage_tile<float, kB, 2 * decltype(t)::value + 1>(), k0, K, k0 + kBK32 <= K);
+    };
+    float fa[2][TM][4], fb[2][TN][4];
+    auto read = [&](int slot, const float* la, const float* lb, int q) __attribute__((always_inline)) {
+        read32<BM, A_KC, TM>(fa[slot], la, wm * 64, q, lane);
+        read32<BN, B_KC, TN>(fb[slot], lb, wn * (BN / 2), q, lane);
+    };
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = f32x4{};
+    auto slice = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[slot][j][e], fa[slot][i][e], acc[i][j], 0, 0, 0);
+    };
+    auto step = [&](auto t, uint32_t s) __attribute__((always_inline)) {
+        constexpr int T = decltype(t)::value;
+        constexpr int U = T ^ 1;
+        read(1, stage_tile<float, kA, 2 * T>(), stage_tile<float, kB, 2 * T + 1>(), 1);
+        slice(0);
+        weave16<kSteps / 4, 4, kReads, 0, kSteps / 8>();
+        __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0(0));  // step s + 1 is in LDS; stage T is read
+        bare_barrier();
+        stage_of(t, s + 2);
+        read(0, stage_tile<float, kA, 2 * U>(), stage_tile<float, kB, 2 * U + 1>(), 0);
+        slice(1);
+        weave16<kSteps / 4, 4, kReads, kLoads, kSteps / 8>();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    stage_of(std::integral_constant<int, 0>{}, 0);
+    stage_of(std::integral_constant<int, 1>{}, 1);
+    __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0(kLoads));  // step 0 is in LDS
+    bare_barrier();
+    read(0, stage_tile<float, kA, 0>(), stage_tile<float, kB, 1>(), 0);
+    for (uint32_t s = 0; s + 1 < steps; s += 2) {
+        step(std::integral_constant<int, 0>{}, s);
+        step(std::integral_constant<int, 1>{}, s + 1);
+    }
+    if (steps % 2 != 0) step(std::integral_constant<int, 0>{}, steps - 1);
+
+    // A lane's results: row `row_of(i)` of the tile and, per run r, kRun
+    // consecutive columns from `col_of(r)` on, column c of it at value(i, r, c).
+    const int x = lane % 16, g = lane / 16;
+    constexpr int kRun = B_KC ? 4 : TN, kRuns = B_KC ? TN : 4;
+    auto row_of = [&](int i) { return static_cast<uint32_t>(wm * 64 + (A_KC ? 16 * i + x : TM * x + i)); };
+    auto col_of = [&](int r) {
+        return static_cast<uint32_t>(wn * (BN / 2) + (B_KC ? 16 * r + 4 * g : TN * (4 * g + r)));
+    };
+    auto value = [&](int i, int r, int c) { return B_KC ? acc[i][r][c] : acc[i][c][r]; };
+    if constexpr (EPI::kProgram) {
+        // The four stage arrays hold the whole tile, 32 rows each.
+        static_assert(BN == 128 && kRun == 4, "runs of four columns, staged whole");
+        constexpr int kRegionRows = kA / BN;
+        float* r0 = stage_tile<float, kA, 0>();
+        float* r1 = stage_tile<float, kB, 1>();
+        float* r2 = stage_tile<float, kA, 2>();
+        float* r3 = stage_tile<float, kB, 3>();
+        // The run form loads what every row reads alike for the thread's
+        // four columns before any store, so no load waits behind one.
+        typename RunState<EPI>::Invariant inv{};
+        if constexpr (HasRuns<EPI>::value) {
+            static_assert(kThreads % (BN / 4) == 0, "a thread keeps its columns in every round");
+            const uint32_t col = n0 + (threadIdx.x % (BN / 4)) * 4;
+            epi.invariant(inv, col < N, col);
+        }
+        __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0(0));  // the last steps' reloads have landed
+        lds_barrier();                               // every wave is done with LDS
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+#pragma unroll
+            for (int r = 0; r < kRuns; r++) {
+                *reinterpret_cast<f32x4*>(staged_at<BN, 0, kRegionRows>(r0, r1, r2, r3, row_of(i), col_of(r))) =
+                    f32x4{value(i, r, 0), value(i, r, 1), value(i, r, 2), value(i, r, 3)};
+            }
+        }
+        lds_barrier();
+        if constexpr (HasRuns<EPI>::value) {
+            program_runs<BN, 0, kRegionRows, BM, BM>(epi, inv, r0, r1, r2, r3, BM, 0, m0, n0, M, N);
+        } else {
+            program_pass<BN, 0, kRegionRows, BM, BM>(epi, r0, r1, r2, r3, BM, 0, m0, n0, M, N);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            const uint32_t row = m0 + row_of(i);
+            if (row >= M) continue;
+            O* to = C + static_cast<uint64_t>(row) * N;
+#pragma unroll
+            for (int r = 0; r < kRuns; r++) {
+                const uint32_t col = n0 + col_of(r);
+                if (!accumulate && col + kRun <= N) {
+                    O out[kRun];
+#pragma unroll
+                    for (int c = 0; c < kRun; c++) out[c] = Elem<O>::narrow(value(i, r, c));
+                    __builtin_memcpy(to + col, out, sizeof(out));
+                } else {
+#pragma unroll
+                    for (int c = 0; c < kRun; c++) {
+                        if (col + c < N) store_out(to, col + c, value(i, r, c), accumulate);
+                    }
+                }
+            }
+        }
+        // No direct load may still be writing LDS when the block ends.
+        __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0(0));
+    }
+}
+
 // C (+)= A . B on 256 x 256 tiles, one tile a block, finished by plain
 // stores or a program epilogue (how a tile is finished, above).  Operands are
 // 16-byte aligned row by row and under 2^31 bytes.
@@ -1015,8 +1077,8 @@ __global__ void __launch_bounds__(512) gemm16x16_kernel(const S* __restrict__ A,
 
     StagerA sa;
     StagerB sb;
-    sa.init(A, m0, M, A_KC ? K : M, K, wave, lane);
-    sb.init(B, n0, N, B_KC ? K : N, K, wave, lane);
+    sa.init(A, m0, M, row_a(epi, A_KC ? K : M), K, wave, lane);
+    sb.init(B, n0, N, row_b(epi, B_KC ? K : N), K, wave, lane);
 
     // Fragment offsets: K-contiguous operands one per slice, row-contiguous
     // ones one per 16-wide block.
@@ -1205,8 +1267,8 @@ __global__ void __launch_bounds__(512) gemm16x16_persistent_kernel(const S* __re
 
     StagerA sa;
     StagerB sb;
-    sa.init(A, m0, M, A_KC ? K : M, K, wave, lane);
-    sb.init(B, n0, N, B_KC ? K : N, K, wave, lane);
+    sa.init(A, m0, M, row_a(epi, A_KC ? K : M), K, wave, lane);
+    sb.init(B, n0, N, row_b(epi, B_KC ? K : N), K, wave, lane);
 
     uint32_t a_off[A_KC ? 2 : TM], b_off[B_KC ? 2 : TN];
     if constexpr (A_KC) {
@@ -1298,8 +1360,8 @@ __global__ void __launch_bounds__(512) gemm16x16_persistent_kernel(const S* __re
                 const uint32_t next = tile + gridDim.x < tiles ? tile + gridDim.x : tile;
                 uint32_t nm, nn;
                 tile_of(next, tiles_m, tiles_n, nm, nn);
-                sa.retarget(A, nm * BM, M, A_KC ? K : M, K);
-                sb.retarget(B, nn * BN, N, B_KC ? K : N, K);
+                sa.retarget(A, nm * BM, M, row_a(epi, A_KC ? K : M), K);
+                sb.retarget(B, nn * BN, N, row_b(epi, B_KC ? K : N), K);
                 k_next = 0;
             }
             step(std::integral_constant<int, 0>{}, k_next);
@@ -1515,8 +1577,8 @@ __global__ void __launch_bounds__(256) gemm16x16_wide_kernel(const S* __restrict
 
     StagerA sa;
     StagerB sb;
-    sa.init(A, m0, M, A_KC ? K : M, K, wave, lane);
-    sb.init(B, n0, N, B_KC ? K : N, K, wave, lane);
+    sa.init(A, m0, M, row_a(epi, A_KC ? K : M), K, wave, lane);
+    sb.init(B, n0, N, row_b(epi, B_KC ? K : N), K, wave, lane);
 
     uint32_t a_off[A_KC ? 2 : TM], b_off[B_KC ? 2 : TN];
     if constexpr (A_KC) {
@@ -1616,8 +1678,8 @@ __global__ void __launch_bounds__(256) gemm16x16_wide_kernel(const S* __restrict
                 const uint32_t next = tile + gridDim.x < tiles ? tile + gridDim.x : tile;
                 uint32_t nm, nn;
                 tile_of(next, tiles_m, tiles_n, nm, nn);
-                sa.retarget(A, nm * BM, M, A_KC ? K : M, K);
-                sb.retarget(B, nn * BN, N, B_KC ? K : N, K);
+                sa.retarget(A, nm * BM, M, row_a(epi, A_KC ? K : M), K);
+                sb.retarget(B, nn * BN, N, row_b(epi, B_KC ? K : N), K);
                 k_next = 0;
             }
             step(std::integral_constant<int, 0>{}, k_next);
