@@ -24,8 +24,10 @@
 // f32 operands (v_mfma_f32_16x16x4_f32, the in-place f32 kernel) are read in
 // place the same way, in 128 x 128 or 128 x 64 tiles and 32-deep steps.
 //
-// Products too small to give those tiles to most CUs, and operands whose rows
-// are not 16-byte aligned, take the register-fed kernel (gemm_sliced.hpp).
+// Products too small to give those tiles to most CUs take the register-fed
+// kernel (gemm_sliced.hpp), which reads operands from any address; operands of
+// larger ones whose rows are not 16-byte aligned are copied to rows that are
+// (gemm_padded.hip), or take that kernel where there is no room to.
 //
 // Operands past 2^31 bytes take the general kernels: both operands
 // K-contiguous, one stored the other way round first transposed into a
@@ -339,37 +341,6 @@ void launch_tiled16(const S* a, const S* b, O* c, uint32_t m, uint32_t k, uint32
     }
 }
 
-// The in-place f32 kernel, in 128 x 128 or 128 x 64 tiles (`narrow32`).
-template <typename O, bool A_KC, bool B_KC, class EPI = PlainStore>
-void launch_inplace32(const float* a, const float* b, O* c, uint32_t m, uint32_t k, uint32_t n, bool accumulate,
-                      hipStream_t s, const EPI& epi = EPI{}) {
-    const uint32_t tiles = ((m + 127) / 128) * ((n + 127) / 128), narrow = ((m + 127) / 128) * ((n + 63) / 64);
-    if constexpr (!EPI::kProgram) {
-        if (narrow32(m, n)) {
-            inplace32_kernel<O, A_KC, B_KC, 128, 64, EPI><<<narrow, kThreads, 0, s>>>(a, b, c, m, n, k, accumulate,
-                                                                                     epi);
-            return;
-        }
-    }
-    inplace32_kernel<O, A_KC, B_KC, 128, 128, EPI><<<tiles, kThreads, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
-}
-
-// ---- register-fed products (gemm_rules.hpp says which) ---------------------------------
-
-template <typename S, typename O, bool A_KC, bool B_KC, class EPI = PlainStore>
-void launch_sliced(const S* a, const S* b, O* c, uint32_t m, uint32_t k, uint32_t n, bool accumulate, hipStream_t s,
-                   const EPI& epi = EPI{}) {
-    const uint32_t tile = sliced_tile(m, n);
-    const uint32_t blocks = ((m + tile - 1) / tile) * ((n + tile - 1) / tile);
-    if (tile == 64) {
-        sliced_kernel<S, O, A_KC, B_KC, 4, 4, 4, 1, EPI><<<blocks, 256, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
-    } else if (tile == 32) {
-        sliced_kernel<S, O, A_KC, B_KC, 2, 2, 4, 1, EPI><<<blocks, 256, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
-    } else {
-        sliced_kernel<S, O, A_KC, B_KC, 1, 1, 8, 4, EPI><<<blocks, 512, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
-    }
-}
-
 // ---- products over a short K -----------------------------------------------------------
 //
 // A product with K below 8 (an outer product, K = 1, is how the tape
@@ -495,15 +466,23 @@ int matmul_typed(uint32_t transposed, bool accumulate, uint64_t m, uint64_t k, u
     }
     // The tiled kernels read operands in place whenever their rows are 16-byte
     // aligned (A is K-contiguous unless LEFT, B only when RIGHT) and stay
-    // under the buffer offsets' 2^31 bytes; small products, and other
-    // operands, take the register-fed kernel.
+    // under the buffer offsets' 2^31 bytes; small products take the
+    // register-fed kernel, and other operands are copied to aligned rows where
+    // that is worth it.
     const bool a_kc = transposed != TC_LEFT, b_kc = transposed == TC_RIGHT;
     constexpr uint64_t kRun = 16 / sizeof(S);
     const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
     if (sliced_reach(m, k, n, sizeof(S))) {
         O* pc = static_cast<O*>(c);
         const bool in_place = aligned16(a) && aligned16(b) && (a_kc ? k : m) % kRun == 0 && (b_kc ? k : n) % kRun == 0;
-        if (!in_place || small_product(m32, n32, std::is_same<S, float>::value)) {
+        const bool small = small_product(m32, n32, std::is_same<S, float>::value);
+        if (!in_place) {
+            bool done = false;
+            const int status = padded_product(Elem<S>::dtype, Elem<O>::dtype, transposed, accumulate, m, k, n, a, b, c,
+                                              s, &done);
+            if (done) return status;
+        }
+        if (!in_place || small) {
             if (a_kc && b_kc) {
                 launch_sliced<S, O, true, true>(pa, pb, pc, m32, k32, n32, accumulate, s);
             } else if (a_kc) {

@@ -787,26 +787,29 @@ __device__ __forceinline__ void weave16() {
     }
 }
 
-// Four consecutive columns of C from a lane's accumulators, (+)=, rounded once
-// (`at` aligned to four elements).
+// Four consecutive columns of C from a lane's accumulators, (+)=, rounded once;
+// one store wherever C's rows start (it may be aligned to an element only).
 template <typename O>
 __device__ __forceinline__ void store_quad(O* at, f32x4 v, bool accumulate) {
     using E = Elem<O>;
     if constexpr (sizeof(O) == 4) {
-        if (accumulate) v += *reinterpret_cast<const f32x4*>(at);
-        *reinterpret_cast<f32x4*>(at) = v;
+        if (accumulate) {
+            f32x4 old;
+            __builtin_memcpy(&old, at, 16);
+            v += old;
+        }
+        __builtin_memcpy(at, &v, 16);
     } else {
         if (accumulate) {
-            const uint2 old = *reinterpret_cast<const uint2*>(at);
-            v[0] += E::widen(__builtin_bit_cast(O, static_cast<uint16_t>(old.x & 0xffff)));
-            v[1] += E::widen(__builtin_bit_cast(O, static_cast<uint16_t>(old.x >> 16)));
-            v[2] += E::widen(__builtin_bit_cast(O, static_cast<uint16_t>(old.y & 0xffff)));
-            v[3] += E::widen(__builtin_bit_cast(O, static_cast<uint16_t>(old.y >> 16)));
+            O old[4];
+            __builtin_memcpy(old, at, 8);
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] += E::widen(old[e]);
         }
         uint2 out;
         out.x = pack_pair<O>(v[0], v[1]);
         out.y = pack_pair<O>(v[2], v[3]);
-        *reinterpret_cast<uint2*>(at) = out;
+        __builtin_memcpy(at, &out, 8);
     }
 }
 
@@ -1191,7 +1194,6 @@ __global__ void __launch_bounds__(512) gemm16x16_kernel(const S* __restrict__ A,
         }
         return;
     }
-    const bool quads = (N % 4) == 0 && (reinterpret_cast<uint64_t>(C) % (4 * sizeof(O))) == 0;
     const uint32_t row0 = m0 + wm * (BM / WM) + lane % 16;
     const uint32_t col0 = n0 + wn * (BN / WN) + 4 * (lane / 16);
     O* base = C + static_cast<uint64_t>(row0) * N + col0;
@@ -1201,7 +1203,7 @@ __global__ void __launch_bounds__(512) gemm16x16_kernel(const S* __restrict__ A,
         for (int j = 0; j < TN; j++) {
             const uint32_t row = row0 + 16 * i, col = col0 + 16 * j;
             O* at = base + static_cast<uint64_t>(16 * i) * N + 16 * j;
-            if (quads && row < M && col + 4 <= N) {
+            if (row < M && col + 4 <= N) {
                 store_quad(at, acc[i][j], accumulate);
             } else if (row < M) {
 #pragma unroll
@@ -1435,7 +1437,6 @@ __global__ void __launch_bounds__(512) gemm16x16_persistent_kernel(const S* __re
             }
           }
         } else {
-            const bool quads = (N % 4) == 0 && (reinterpret_cast<uint64_t>(C) % (4 * sizeof(O))) == 0;
             const uint32_t row0 = m0 + wm * (BM / WM) + lane % 16;
             const uint32_t col0 = n0 + wn * (BN / WN) + 4 * (lane / 16);
             O* base = C + static_cast<uint64_t>(row0) * N + col0;
@@ -1445,7 +1446,7 @@ __global__ void __launch_bounds__(512) gemm16x16_persistent_kernel(const S* __re
                 for (int j = 0; j < TN; j++) {
                     const uint32_t row = row0 + 16 * i, col = col0 + 16 * j;
                     O* at = base + static_cast<uint64_t>(16 * i) * N + 16 * j;
-                    if (quads && row < M && col + 4 <= N) {
+                    if (row < M && col + 4 <= N) {
                         store_quad(at, acc[i][j], accumulate);
                     } else if (row < M) {
 #pragma unroll

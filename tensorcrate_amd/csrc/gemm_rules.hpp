@@ -1,10 +1,12 @@
-// Which kernel and tile a matrix product takes, by its sizes: the rules the
-// product's translation units share.
+// Which kernel and tile a matrix product takes, by its sizes: the rules, and the
+// launches, that the product's translation units share.
 #pragma once
 
 #include <algorithm>
 
 #include "common.hpp"
+#include "gemm_kernels.hpp"
+#include "gemm_sliced.hpp"
 
 namespace tc {
 
@@ -57,5 +59,79 @@ inline bool narrow32(uint32_t m, uint32_t n) {
     const uint64_t wide = rows * ((n + 127) / 128), narrow = rows * ((n + 63) / 64);
     return (narrow + cus - 1) / cus * 21 < (wide + cus - 1) / cus * 40;
 }
+
+// Whether operands that the tiled kernels cannot read in place are worth
+// copying for one.  us a call, register-fed kernel / copies and tiled kernel:
+//  - 16-bit, an operand along K: the register-fed kernel's odd loads along K are
+//    slow, and the copies' few microseconds are made up from about 2^28
+//    multiplications: (A along K) 1153 x 33 x 1153 4.9 / 8.1, 2047 x 17 x 2047 9.1 /
+//    10.1, 1153 x 255 x 1153 13.3 / 10.8, 2047 x 1001 x 1531 38 / 26, 4097^3 1041 /
+//    206; (both) 5.6 / 8.0, 9.9 / 9.9, 19.8 / 10.5, 54 / 27, 1653 / 205.
+//  - 16-bit, neither: from about 2^32: 1153 x 1025 x 1153 16.8 / 23.5, 2047 x 1001
+//    x 1531 24.0 / 24.6, 1025 x 4095 x 2047 72 / 61, 4097^3 413 / 207.
+//  - f32, whose matrix cores hide those loads better: where the tiles' last
+//    rounds and edges leave the CUs four sevenths of a whole product's work
+//    (65 x 2049 x 20481, a third: 130 / 173; 1025 x 4095 x 2047, half: 246 / 252;
+//    1153 x 1025 x 1153, 0.6: 49 / 48; 2047 x 1001 x 1531, 0.75: 84 / 76; 4097^3
+//    1433 / 1093), from 2^30 (1153 x 255 x 1153 16.4 / 17.5).
+inline bool worth_tiled_copies(uint32_t m, uint32_t k, uint32_t n, bool f32, bool along_k) {
+    const uint64_t work = static_cast<uint64_t>(m) * n * k;
+    if (!f32) return work >= (along_k ? uint64_t{1} << 28 : uint64_t{1} << 32);
+    const uint64_t cus = static_cast<uint64_t>(compute_units()), rows = (m + 127) / 128;
+    const uint64_t wide = rows * ((n + 127) / 128), narrow = rows * ((n + 63) / 64);
+    const uint64_t rounds = std::min((narrow + cus - 1) / cus * 21, (wide + cus - 1) / cus * 40);
+    return work >= uint64_t{1} << 30 &&
+           rounds * cus * 128 * 128 * 4 <= 7 * 40 * static_cast<uint64_t>(m) * n;
+}
+
+// Whether a small 16-bit product's odd operands along K are worth copying for the
+// register-fed kernel: what the copies' few microseconds win is the chain of odd
+// loads along K, which that kernel's 16 x 16 tiles cut into more pieces.  us a
+// call, as they are / copied, A along K and both: 1023 x 511 x 1023 12.3 / 10.9 and
+// 18.1 / 13.2, 101 x 501 x 8191 9.5 / 9.3 and 12.1 / 15.5, 700 x 701 x 699 10.6 /
+// 11.0 and 14.1 / 13.2, 333 x 777 x 555 8.2 / 8.1 and 10.2 / 9.1, 511 x 1001 x 511
+// 9.0 / 8.8 and 11.8 / 9.3, 1023 x 4095 x 1023 65 / 38 and 102 / 44; in 16 x 16
+// tiles 255 x 1001 x 255 5.2 / 7.7 and 6.7 / 8.0, 255 x 2049 x 255 13.2 / 11.4 and
+// 20.1 / 9.4, 16 x 2049 x 4097 28.7 / 22.9 and 29.5 / 14.9.
+inline bool worth_sliced_copies(uint32_t m, uint32_t k, uint32_t n) {
+    return k >= (sliced_tile(m, n) == 16 ? 2048 : 768);
+}
+
+// The in-place f32 kernel, in 128 x 128 or 128 x 64 tiles (`narrow32`).
+template <typename O, bool A_KC, bool B_KC, class EPI = PlainStore>
+void launch_inplace32(const float* a, const float* b, O* c, uint32_t m, uint32_t k, uint32_t n, bool accumulate,
+                      hipStream_t s, const EPI& epi = EPI{}) {
+    const uint32_t tiles = ((m + 127) / 128) * ((n + 127) / 128), narrow = ((m + 127) / 128) * ((n + 63) / 64);
+    if constexpr (!EPI::kProgram) {
+        if (narrow32(m, n)) {
+            inplace32_kernel<O, A_KC, B_KC, 128, 64, EPI><<<narrow, kThreads, 0, s>>>(a, b, c, m, n, k, accumulate,
+                                                                                     epi);
+            return;
+        }
+    }
+    inplace32_kernel<O, A_KC, B_KC, 128, 128, EPI><<<tiles, kThreads, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
+}
+
+// The sliced kernel, in its tile for the product.
+template <typename S, typename O, bool A_KC, bool B_KC, class EPI = PlainStore>
+void launch_sliced(const S* a, const S* b, O* c, uint32_t m, uint32_t k, uint32_t n, bool accumulate, hipStream_t s,
+                   const EPI& epi = EPI{}) {
+    const uint32_t tile = sliced_tile(m, n);
+    const uint32_t blocks = ((m + tile - 1) / tile) * ((n + tile - 1) / tile);
+    if (tile == 64) {
+        sliced_kernel<S, O, A_KC, B_KC, 4, 4, 4, 1, EPI><<<blocks, 256, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
+    } else if (tile == 32) {
+        sliced_kernel<S, O, A_KC, B_KC, 2, 2, 4, 1, EPI><<<blocks, 256, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
+    } else {
+        sliced_kernel<S, O, A_KC, B_KC, 1, 1, 8, 4, EPI><<<blocks, 512, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
+    }
+}
+
+// The product as `tc_matmul` forms it, of operands the tiled kernels cannot read
+// in place, which are first copied to rows of whole 16-byte words
+// (gemm_padded.hip).  `*done` is false, with nothing launched, where that is not
+// worth it, or the copies would pass the kernels' 2^31 bytes or have no memory.
+int padded_product(uint32_t in_dtype, uint32_t out_dtype, uint32_t transposed, bool accumulate, uint64_t m, uint64_t k,
+                   uint64_t n, const void* a, const void* b, void* c, hipStream_t s, bool* done);
 
 }  // namespace tc

@@ -205,7 +205,8 @@ __device__ __forceinline__ void settle(uint4 (&fa)[VA], uint4 (&fb)[VB]) {
 // f32 512^3 24.2 / 5.8, f32 1024^3 44.9 / 22.4, f32 256 x 8192 x 256 327 / 27,
 // bf16 1024^3 14.8 / 9.3, bf16 16 x 4096 x 4096 with B transposed 42.4 / 11.1;
 // operands whose rows are not 16-byte aligned, which the tiled kernels cannot
-// read: bf16 2047 x 1001 x 1531 258 / 38, f32 424 / 75.  At 2048 x 1024 x 1536
+// read: f32 1153 x 255 x 1153 16.4 (17.5 with copies), bf16 1023 x 255 x 1023 8.4
+// (9.1).  At 2048 x 1024 x 1536
 // aligned it is past its range: bf16 15.5 / 21.8, the waves' rereading of
 // their operands from L2 then costing more than the tiled kernel's barriers.
 template <typename S, typename O, bool A_KC, bool B_KC, int VA, int VB, int W, int U, class EPI = PlainStore>
@@ -222,8 +223,8 @@ __global__ void __launch_bounds__(W * 64) sliced_kernel(const S* __restrict__ A,
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     OA a;
     OB b;
-    a.init(A, tm * 16 * VA, M, A_KC ? K : M, lane);
-    b.init(B, tn * 16 * VB, N, B_KC ? K : N, lane);
+    a.init(A, tm * 16 * VA, M, row_a(epi, A_KC ? K : M), lane);
+    b.init(B, tn * 16 * VB, N, row_b(epi, B_KC ? K : N), lane);
 
     f32x4 acc[VA][VB];
 #pragma unroll
