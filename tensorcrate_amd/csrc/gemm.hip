@@ -335,9 +335,7 @@ void launch_tiled16(const S* a, const S* b, O* c, uint32_t m, uint32_t k, uint32
         }
         gemm16x16_kernel<S, O, A_KC, B_KC, EPI><<<large, 512, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
     } else {
-        const uint32_t small = ((m + 127) / 128) * ((n + 127) / 128);
-        direct16_kernel<S, O, A_KC, B_KC, 128, 128, 2, 2, 64, 2, EPI><<<small, 2 * 2 * 64, 0, s>>>(a, b, c, m, n, k,
-                                                                                                 accumulate, epi);
+        launch_direct16<S, O, A_KC, B_KC>(a, b, c, m, k, n, accumulate, s, epi);
     }
 }
 

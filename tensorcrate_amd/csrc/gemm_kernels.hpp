@@ -322,21 +322,27 @@ __device__ __forceinline__ void weave() {
 //    lives at chunk c ^ ((r / RPW) % CPR), which spreads the 16 rows a
 //    ds_read_b128 phase touches over all 16 bank groups.
 //  - row-contiguous tile, ROWS x 2-byte rows: chunk c of k-row r lives at
-//    c ^ ((r & 3) << 2), which spreads the four rows of a transposing read
-//    over distinct bank groups.
+//    c ^ ((r & 3) << 2), or c ^ ((r & 2) << 1) in a 64-wide tile, whose rows are
+//    eight chunks, two to a bank window: either spreads the four rows of a
+//    transposing read over distinct bank groups.
 // The K loop runs NS stages deep: each step issues the loads of the step
 // NS - 1 ahead into the stage the previous step freed, then waits only for
 // the next step's loads (vmcnt counts this wave's loads in issue order).
-// Two 64-deep stages measure faster on MI355X than three or four 32-deep
-// ones (1170 vs 950 TFLOP/s at 8192^3): the per-step barrier costs more
-// than the extra latency cover buys.
+// 64-deep stages measure faster on MI355X than 32-deep ones (two against three
+// or four, 1170 vs 950 TFLOP/s at 8192^3): the per-step barrier costs more than
+// the extra latency cover buys.  Two of them, at 64 KiB for a 128 x 128 tile, let
+// two blocks share a CU and cover each other's loads; a block that has its CU to
+// itself covers them with a third or fourth (launch_direct16).
 
 template <int BK>
 __device__ __forceinline__ int kc_swizzle(int row) {
     constexpr int kCpr = BK / 8, kRpw = 256 / (2 * BK);
     return (row / kRpw) % kCpr;
 }
-__device__ __forceinline__ int rc_swizzle(int row) { return (row & 3) << 2; }
+template <int ROWS>
+__device__ __forceinline__ int rc_swizzle(int row) {
+    return ROWS == 64 ? (row & 2) << 1 : (row & 3) << 2;
+}
 
 template <typename S, int ROWS, bool KC, int WAVES, int BK>
 struct DirectStager {
@@ -369,7 +375,7 @@ struct DirectStager {
             const int first_row = kRowsPer * (w + WAVES * i);
             const int row = first_row + lane / kChunksPerRow;
             const int place = lane % kChunksPerRow;
-            const int chunk = place ^ (KC ? kc_swizzle<BK>(row) : rc_swizzle(row));
+            const int chunk = place ^ (KC ? kc_swizzle<BK>(row) : rc_swizzle<ROWS>(row));
             offset[i] = (static_cast<uint32_t>(row) * ld + chunk * 8) * sizeof(S);
             k_of[i] = KC ? chunk * 8 : 0;
         }
@@ -412,7 +418,7 @@ __device__ __forceinline__ uint4 swizzled_fragment(const S* lds, int row_base, i
         const int g = lane / 16, j = lane % 16;
         const int k = k_base + (g / 2) * 8 + j / 4;
         const int col = row_base + (g % 2) * 16 + 4 * (j % 4);
-        const int chunk = (col / 8) ^ rc_swizzle(k);  // k + 4 swizzles the same way
+        const int chunk = (col / 8) ^ rc_swizzle<ROWS>(k);  // k + 4 swizzles the same way
         const S* at = lds + k * ROWS + chunk * 8 + col % 8;
         short4v lo = read_tr16(at);
         short4v hi = read_tr16(at + 4 * ROWS);
@@ -425,9 +431,30 @@ __device__ __forceinline__ uint4 swizzled_fragment(const S* lds, int row_base, i
     }
 }
 
-// s_waitcnt's immediate for vmcnt(n), other counters not waited on
-// (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
-constexpr int vmcnt_wait(int n) { return (n & 0xf) | ((n >> 4) << 14) | (0x7 << 4) | (0xf << 8); }
+// s_waitcnt immediates: vmcnt(n) and lgkmcnt(0); lgkmcnt(0) alone.
+constexpr int vmcnt_lgkm0(int n) { return (n & 0xf) | ((n >> 4) << 14) | (0x7 << 4); }
+
+// A workgroup barrier that orders nothing by itself: callers wait for what
+// they need first.  The compiler keeps memory accesses on their side.
+__device__ __forceinline__ void bare_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// The barrier at which all but this wave's last `LOADS` direct loads are in LDS
+// and its LDS reads are done.  __syncthreads' fence waits for every load.
+template <int LOADS>
+__device__ __forceinline__ void staged_barrier() {
+    if constexpr (LOADS == 0) {
+        __syncthreads();
+    } else {
+        __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0(LOADS));
+        bare_barrier();
+    }
+}
 
 // One LDS stage of an operand.  A separate array per stage gives every LDS
 // read and every direct load a distinct, statically known object, so the
@@ -509,8 +536,7 @@ __global__ void __launch_bounds__(WM * WN * 64) direct16_kernel(const S* __restr
                 for (int j = 0; j < TN; j++) acc[i][j] = Mfma16<S>::step(fa[q & 1][i], fb[q & 1][j], acc[i][j]);
         }
         weave<kSteps, kLoads, kReads, kSlices - 1>();
-        __builtin_amdgcn_s_waitcnt(vmcnt_wait(kLoads * (NS - 2)));  // step s + 1 is in LDS
-        __syncthreads();
+        staged_barrier<kLoads * (NS - 2)>();  // step s + 1 is in LDS; stage T is read
         constexpr int last = (kSlices - 1) & 1;
         constexpr int U = (T + 1) % NS;
         read_fragments(last ^ 1, stage_tile<S, kA, 2 * U>(), stage_tile<S, kB, 2 * U + 1>(), 0);
@@ -524,8 +550,7 @@ __global__ void __launch_bounds__(WM * WN * 64) direct16_kernel(const S* __restr
         stage_of(std::integral_constant<int, 0>{}, 0);
         if constexpr (NS > 2) stage_of(std::integral_constant<int, 1>{}, 1);
         if constexpr (NS > 3) stage_of(std::integral_constant<int, 2>{}, 2);
-        __builtin_amdgcn_s_waitcnt(vmcnt_wait(kLoads * (NS - 2)));  // step 0 is in LDS
-        __syncthreads();
+        staged_barrier<kLoads * (NS - 2)>();  // step 0 is in LDS
         read_fragments(0, stage_tile<S, kA, 0>(), stage_tile<S, kB, 1>(), 0);
     }
     for (uint32_t s = 0; s < steps; s += NS) {
@@ -542,7 +567,7 @@ __global__ void __launch_bounds__(WM * WN * 64) direct16_kernel(const S* __restr
     if constexpr (EPI::kProgram) {
         // The four stage arrays, BK / 2 rows of BN floats each, hold a pass
         // of 2 BK rows.
-        static_assert(NS == 2 && BM == BN && kA == kB, "square tiles over two stages");
+        static_assert(BM == BN && kA == kB, "square tiles over the first two stages");
         constexpr int kRegionRows = kA * static_cast<int>(sizeof(S)) / 4 / BN;
         constexpr int kPass = 4 * kRegionRows;
         constexpr int kPasses = BM / kPass, H = BM / WM / kPasses;
@@ -551,7 +576,7 @@ __global__ void __launch_bounds__(WM * WN * 64) direct16_kernel(const S* __restr
         float* r1 = reinterpret_cast<float*>(stage_tile<S, kB, 1>());
         float* r2 = reinterpret_cast<float*>(stage_tile<S, kA, 2>());
         float* r3 = reinterpret_cast<float*>(stage_tile<S, kB, 3>());
-        __builtin_amdgcn_s_waitcnt(vmcnt_wait(0));  // the last step's reload has landed
+        __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0(0));  // the last steps' reloads have landed
 #pragma unroll
         for (int pass = 0; pass < kPasses; pass++) {
             lds_barrier();  // every wave is done with LDS
@@ -601,7 +626,10 @@ __global__ void __launch_bounds__(WM * WN * 64) direct16_kernel(const S* __restr
             }
         }
     }
+    // No direct load may still be writing LDS when the block ends.
+    if constexpr (NS > 2) __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0(0));
 }
+
 // ---- the 16 x 16 x 32 kernel ---------------------------------------------------
 //
 // The large-product kernel: 256 x 256 block tiles over eight waves of 128 x 64
@@ -644,19 +672,6 @@ struct Mfma16x16<_Float16> {
                                                       0, 0);
     }
 };
-
-// s_waitcnt immediates: vmcnt(n) and lgkmcnt(0); lgkmcnt(0) alone.
-constexpr int vmcnt_lgkm0(int n) { return (n & 0xf) | ((n >> 4) << 14) | (0x7 << 4); }
-
-// A workgroup barrier that orders nothing by itself: callers wait for what
-// they need first.  The compiler keeps memory accesses on their side.
-__device__ __forceinline__ void bare_barrier() {
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-}
 
 // Chunk swizzle of a row-contiguous tile for the 16 x 16 x 32 reads: k-rows 0-3
 // and 8-11 of a slice (one half-wave's transposing read) differ in the low

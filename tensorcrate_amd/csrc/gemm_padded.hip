@@ -5,7 +5,7 @@
 // the copies, C written where it belongs.
 //
 // The copy is bandwidth-bound and both operands' go in one launch: 5.6 us of the
-// 25.6 at bf16 2047 x 1001 x 1531 (14 MB), 20.4 of 206 at 4097^3 (6.5 TB/s); it grows
+// 22.3 at bf16 2047 x 1001 x 1531 (14 MB), 20.4 of 206 at 4097^3 (6.5 TB/s); it grows
 // with the sides where the product grows with the sides times K.  gemm_rules.hpp
 // has the lines between these, with both sides' times.
 
@@ -79,8 +79,7 @@ void launch(Kernel kernel, const S* a, const S* b, O* c, uint32_t m, uint32_t k,
         gemm16x16_persistent_kernel<S, O, A_KC, B_KC, PaddedStore>
             <<<compute_units(), 512, 0, s>>>(a, b, c, m, n, k, accumulate, store);
     } else if (kernel == Kernel::tiled) {
-        direct16_kernel<S, O, A_KC, B_KC, 128, 128, 2, 2, 64, 2, PaddedStore>
-            <<<((m + 127) / 128) * ((n + 127) / 128), 256, 0, s>>>(a, b, c, m, n, k, accumulate, store);
+        launch_direct16<S, O, A_KC, B_KC>(a, b, c, m, k, n, accumulate, s, store);
     } else if constexpr (A_KC) {
         launch_sliced<S, O, A_KC, B_KC>(a, b, c, m, k, n, accumulate, s, store);
     }

@@ -60,14 +60,45 @@ inline bool narrow32(uint32_t m, uint32_t n) {
     return (narrow + cus - 1) / cus * 21 < (wide + cus - 1) / cus * 40;
 }
 
+// The 16-bit tiled kernel for products of fewer 256 x 256 tiles than CUs.  A step's
+// loads take longer to land (some 0.6 us) than its matrix-core steps (0.2), so
+// what bounds it is how many loads a CU keeps in flight: two blocks of two stages
+// where there are tiles for that, else one block of more stages, in 128 x 64 tiles
+// while those are no more than the CUs.  us a call, two stages / three / 128 x 64
+// and four: 1152 x 4096 x 1152, 162 narrow tiles, 46.3 / 36.3 / 26.4 (B transposed
+// 44.4 / 31.8 / 24.9); 1280 x 1024 x 1280, 200, 11.7 / 10.9 / 9.5; (B transposed) 2048^3,
+// 512, 27.3 / 20.9 / 27.7; 4096 x 1024 x 2048, 1024, 21.1 / 22.5 / 29.3.  The order of
+// the sums is the same in all.  A program's epilogue keeps the one shape it is
+// compiled for.
+template <typename S, typename O, bool A_KC, bool B_KC, class EPI = PlainStore>
+void launch_direct16(const S* a, const S* b, O* c, uint32_t m, uint32_t k, uint32_t n, bool accumulate, hipStream_t s,
+                     const EPI& epi = EPI{}) {
+    const uint32_t cus = static_cast<uint32_t>(compute_units()), rows = (m + 127) / 128;
+    const uint32_t wide = rows * ((n + 127) / 128), narrow = rows * ((n + 63) / 64);
+    if constexpr (!EPI::kProgram) {
+        if (narrow <= cus) {
+            direct16_kernel<S, O, A_KC, B_KC, 128, 64, 2, 2, 64, 4, EPI><<<narrow, 256, 0, s>>>(a, b, c, m, n, k,
+                                                                                             accumulate, epi);
+            return;
+        }
+        if (wide <= cus) {
+            direct16_kernel<S, O, A_KC, B_KC, 128, 128, 2, 2, 64, 3, EPI><<<wide, 256, 0, s>>>(a, b, c, m, n, k,
+                                                                                            accumulate, epi);
+            return;
+        }
+    }
+    direct16_kernel<S, O, A_KC, B_KC, 128, 128, 2, 2, 64, 2, EPI><<<wide, 256, 0, s>>>(a, b, c, m, n, k, accumulate,
+                                                                                    epi);
+}
+
 // Whether operands that the tiled kernels cannot read in place are worth
 // copying for one.  us a call, register-fed kernel / copies and tiled kernel:
 //  - 16-bit, an operand along K: the register-fed kernel's odd loads along K are
 //    slow, and the copies' few microseconds are made up from about 2^28
 //    multiplications: (A along K) 1153 x 33 x 1153 4.9 / 8.1, 2047 x 17 x 2047 9.1 /
-//    10.1, 1153 x 255 x 1153 13.3 / 10.8, 2047 x 1001 x 1531 38 / 26, 4097^3 1041 /
-//    206; (both) 5.6 / 8.0, 9.9 / 9.9, 19.8 / 10.5, 54 / 27, 1653 / 205.
-//  - 16-bit, neither: from about 2^32: 1153 x 1025 x 1153 16.8 / 23.5, 2047 x 1001
+//    10.1, 1153 x 255 x 1153 13.3 / 10.8, 2047 x 1001 x 1531 38 / 23, 4097^3 1041 /
+//    206; (both) 5.6 / 8.0, 9.9 / 9.9, 19.8 / 10.5, 54 / 23, 1653 / 205.
+//  - 16-bit, neither: from about 2^32: 1153 x 1025 x 1153 16.8 / 16.5, 2047 x 1001
 //    x 1531 24.0 / 24.6, 1025 x 4095 x 2047 72 / 61, 4097^3 413 / 207.
 //  - f32, whose matrix cores hide those loads better: where the tiles' last
 //    rounds and edges leave the CUs four sevenths of a whole product's work
