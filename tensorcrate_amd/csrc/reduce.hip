@@ -811,8 +811,9 @@ int launch_reduce(const S* in, O* out, const Plan& plan, const Finish& f, hipStr
         if (stream) return launch_rows<S, P, O, true, I>(in, out, plan, f, s, what);
         return launch_rows<S, P, O, false, I>(in, out, plan, f, s, what);
     }
-    // Columns: contiguous neighbouring results, one strided folded axis.
-    if (folded.rank == 1 && kept.rank >= 1 && kept.strides[kept.rank - 1] == 1) {
+    // Columns: contiguous neighbouring results, one strided folded axis, not
+    // empty (there is nothing to spread: the general kernel answers).
+    if (depth > 0 && folded.rank == 1 && kept.rank >= 1 && kept.strides[kept.rank - 1] == 1) {
         // An input past the Infinity Cache streams with 16-byte words.  A
         // smaller one takes 4 bytes of columns a lane, which spreads it over
         // four times the threads, and one column for variances and

@@ -6,6 +6,8 @@ bytes.  Extremes and arg-reductions are exact, with NaNs, infinities and ties
 among the values; sums, means and variances are within the bound of
 tests/test_gpu_reduce.py of f64."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,14 @@ def test_extremes_and_arg_reductions_with_specials(kind):
                 want = oracle.arg_reduce(kind, host, list(shape), view.offset, list(view.strides), axes[0], op)
                 got = getattr(view, name)(axes[0]).to_numpy()
                 assert np.array_equal(got, want), (shape, axes, name, view.offset)
+
+
+@pytest.mark.parametrize("columns", [1, 2, 5, 15, 16, 300])
+def test_an_empty_fold_called_directly_gives_the_identity(columns):
+    # Shape [0, columns] folded along axis 0, straight to the library: the
+    # tensor layer answers empty folds itself.
+    source, out = lib.Buffer(16), lib.Buffer(4 * columns)
+    split = lib.split(0, [columns], [1], [0], [columns])
+    for kind, op, want in ((lib.FOLD, lib.SUM, 0.0), (lib.FOLD, lib.RMAX, -np.inf), (lib.FOLD, lib.RMIN, np.inf)):
+        lib.call("tc_reduce_axes", lib.F32, source.ptr, 0, ctypes.byref(split), kind, op, 0, out.ptr)
+        assert np.all(out.download(np.float32, columns) == np.float32(want))
