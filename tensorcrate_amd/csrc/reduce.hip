@@ -844,7 +844,10 @@ int reduce_typed(const void* input, void* out, uint64_t offset, const Plan& plan
     TC_STREAM(s);
     const S* in = static_cast<const S*>(input) + offset;
     if (plan.results == 0) return TC_OK;
-    bool small = plan.results <= UINT32_MAX && plan.depth <= UINT32_MAX && input_len <= UINT32_MAX;
+    // The kernels step past their last row and result by as much as a grid's
+    // whole turn (2^21), which 32-bit indexes must hold too.
+    const uint64_t most = UINT32_MAX / 2;
+    const bool small = plan.results <= most && plan.depth <= most && input_len <= UINT32_MAX;
     if (small) return launch_reduce<S, P, O, uint32_t>(in, static_cast<O*>(out), plan, f, s, what);
     return launch_reduce<S, P, O, uint64_t>(in, static_cast<O*>(out), plan, f, s, what);
 }

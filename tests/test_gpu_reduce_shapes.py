@@ -87,3 +87,10 @@ def test_an_empty_fold_called_directly_gives_the_identity(columns):
     for kind, op, want in ((lib.FOLD, lib.SUM, 0.0), (lib.FOLD, lib.RMAX, -np.inf), (lib.FOLD, lib.RMIN, np.inf)):
         lib.call("tc_reduce_axes", lib.F32, source.ptr, 0, ctypes.byref(split), kind, op, 0, out.ptr)
         assert np.all(out.download(np.float32, columns) == np.float32(want))
+
+
+@pytest.mark.parametrize("depth", [2 ** 31 - 1, 2 ** 31 + 1, 2 ** 32 - 1000])
+def test_depths_whose_steps_pass_32_bits(depth):
+    # Two columns repeated: a lane's rows are 256 apart, eight in flight.
+    view = Tensor.from_numpy(np.array([3.0, -2.0], np.float32)).broadcast_to([depth, 2])
+    assert view.max_axes(0).to_numpy().tolist() == [3.0, -2.0]
