@@ -142,7 +142,7 @@ __global__ void __launch_bounds__(256) rows_kernel(Pieces<I, N> pieces) {
         T* dst = static_cast<T*>(w.dst) + to + at;
         if (PER == 1) {
             *dst = *src;
-        } else if (at + PER <= w.run) {
+        } else if (w.run - at >= PER) {  // at + PER would wrap near the end of I
             store_any_word<false>(dst, load_any_word<NT>(src));
         } else {
             for (I k = 0; k < w.run - at; k++) dst[k] = src[k];

@@ -79,6 +79,26 @@ def test_pieces_that_overlap_are_copied_in_order():
     assert np.array_equal(dst.download(np.float32).reshape(20, 20), want)
 
 
+@pytest.mark.parametrize("dtype,run", [(np.uint8, 2 ** 32 - 1), (np.uint8, 2 ** 32 - 15), (np.uint16, 2 ** 32 - 3)])
+def test_the_last_word_of_a_run_near_2_to_32(dtype, run):
+    # Its first element's index plus a word's elements is past 32 bits.
+    size = np.dtype(dtype).itemsize
+    source, target = lib.Buffer(run * size), lib.Buffer((run + 40) * size)
+    five, nine = np.array([5], dtype), np.array([9], dtype)
+    lib.call("tc_fill", source.ptr, run, size, five.ctypes.data)
+    lib.call("tc_fill", target.ptr, run + 40, size, nine.ctypes.data)
+    end = np.arange(20, 60, dtype=dtype)
+    lib.call("tc_upload", source.ptr + (run - 40) * size, end.ctypes.data, end.nbytes)
+    region = lib.region(source, run, [run], 0, [1], 3, [1])
+    lib.call("tc_strided_write", size, target.ptr, run + 40, lib.ctypes.byref(region))
+    got = np.empty(120, dtype)
+    lib.call("tc_download", got.ctypes.data, target.ptr + (run + 40 - 120) * size, got.nbytes)
+    assert got.tolist() == [5] * 43 + end.tolist() + [9] * 37
+    source.free()
+    target.free()
+    lib.call("tc_empty_cache")
+
+
 @pytest.mark.parametrize("kind", KINDS, ids=[KIND_NAMES[k] for k in KINDS])
 @pytest.mark.parametrize("shape", [(3, 5, 1), (4, 3, 7), (3, 5, 8), (2, 7, 9), (3, 4, 15), (2, 3, 17), (3, 9, 64), (5, 4, 131)])
 def test_broadcasts_over_odd_runs(kind, shape):
