@@ -687,14 +687,25 @@ int launch_combine(const typename P::State* partial, O* out, uint64_t results, u
     return check_launch(what);
 }
 
-// Block states of a split reduction, in a block from the thread's cache.
+// How a depth is cut: `splits` pieces of `per_split` (the last may hold fewer),
+// and where their states go, in a block from the thread's cache, if there is
+// more than one.  Without the memory for that the depth stays whole, which is
+// slower and needs none.
 template <typename State>
-int split_states(uint64_t count, State** partial) {
-    void* scratch = nullptr;
-    const int status = tc_alloc(count * sizeof(State), &scratch);
-    *partial = static_cast<State*>(scratch);
-    return status;
-}
+struct Cut {
+    uint64_t splits, per_split;
+    State* partial = nullptr;
+    Cut(uint64_t depth, uint64_t wanted, uint64_t multiple, uint64_t results) {
+        per_split = wanted < 2 ? depth : (depth + wanted * multiple - 1) / (wanted * multiple) * multiple;
+        splits = (depth + per_split - 1) / per_split;
+        void* scratch = nullptr;
+        if (splits > 1 && tc_alloc(splits * results * sizeof(State), &scratch) != TC_OK) {
+            splits = 1;
+            per_split = depth;
+        }
+        partial = static_cast<State*>(scratch);
+    }
+};
 
 // The columns kernel over a plan whose innermost kept axis is contiguous and
 // whose one folded axis is strided; VC columns per lane.
@@ -722,17 +733,16 @@ int launch_columns(const S* in, O* out, const Plan& plan, const Finish& f, hipSt
     uint64_t splits = 1;
     if (base_blocks * 2 <= want) {
         splits = std::min((want + base_blocks - 1) / base_blocks, depth / (groups * 32));
-        if (splits < 2) splits = 1;
     }
-    const uint64_t per_split = (depth + splits - 1) / splits;
-    splits = (depth + per_split - 1) / per_split;
+    const Cut<typename P::State> cut(depth, splits, 1, results);
+    splits = cut.splits;
     w.columns = static_cast<I>(columns);
     w.depth = static_cast<I>(depth);
     w.step = static_cast<I>(plan.folded.strides[0]);
     w.tiles = static_cast<I>(tiles);
     w.tiles_div.set(tiles);
     w.splits = static_cast<I>(splits);
-    w.per_split = static_cast<I>(per_split);
+    w.per_split = static_cast<I>(cut.per_split);
     w.lanes = static_cast<uint32_t>(lanes);
     w.groups = static_cast<uint32_t>(groups);
     // Rows of under 64 bytes: neighbouring groups on neighbouring rows share
@@ -742,16 +752,14 @@ int launch_columns(const S* in, O* out, const Plan& plan, const Finish& f, hipSt
     w.apart = lanes * VC * sizeof(S) < 64;
     w.lanes_div = DivMod(w.lanes);
     const uint64_t blocks = base_blocks * splits;
-    typename P::State* partial = nullptr;
-    int status = splits > 1 ? split_states(splits * results, &partial) : TC_OK;
-    if (status != TC_OK) return status;
+    typename P::State* partial = cut.partial;
     const uint32_t grid = grid_for(blocks, 1, 64);
     if (lanes == 64 && groups == 4) {
         columns_kernel<S, P, O, VC, true, NT, I><<<grid, 256, 0, s>>>(in, out, partial, w, static_cast<I>(blocks), f);
     } else {
         columns_kernel<S, P, O, VC, false, NT, I><<<grid, 256, 0, s>>>(in, out, partial, w, static_cast<I>(blocks), f);
     }
-    status = check_launch(what);
+    int status = check_launch(what);
     if (status == TC_OK && splits > 1) status = launch_combine<P, O, I>(partial, out, results, splits, f, s, what);
     // Stream order keeps the block alive until both kernels have run.
     if (partial != nullptr) tc_free(partial);
@@ -774,16 +782,13 @@ int launch_rows(const S* in, O* out, const Plan& plan, const Finish& f, hipStrea
     const uint64_t want = static_cast<uint64_t>(compute_units()) * 4, round = 64 * V * 4;
     uint64_t splits = 1;
     if (lanes == 64 && results < want) splits = std::min((want + results - 1) / results, depth / (round * 8));
-    if (splits < 2) splits = 1;
-    const uint64_t per_split = splits == 1 ? depth : (depth + splits * V - 1) / (splits * V) * V;
-    splits = (depth + per_split - 1) / per_split;
+    const Cut<typename P::State> cut(depth, splits, V, results);
+    splits = cut.splits;
     w.splits = static_cast<I>(splits);
-    w.per_split = static_cast<I>(per_split);
+    w.per_split = static_cast<I>(cut.per_split);
     w.splits_div.set(splits);
     w.lanes = static_cast<uint32_t>(lanes);
-    typename P::State* partial = nullptr;
-    int status = splits > 1 ? split_states(splits * results, &partial) : TC_OK;
-    if (status != TC_OK) return status;
+    typename P::State* partial = cut.partial;
     const uint32_t per_block = static_cast<uint32_t>(256 / lanes);
     const uint32_t blocks = grid_for(results * splits, per_block, 32);
     if (lanes < 64) {
@@ -793,7 +798,7 @@ int launch_rows(const S* in, O* out, const Plan& plan, const Finish& f, hipStrea
     } else {
         rows_kernel<S, P, O, Rows::split, NT, I><<<blocks, 256, 0, s>>>(in, out, partial, w, f);
     }
-    status = check_launch(what);
+    int status = check_launch(what);
     if (status == TC_OK && splits > 1) status = launch_combine<P, O, I>(partial, out, results, splits, f, s, what);
     if (partial != nullptr) tc_free(partial);
     return status;
