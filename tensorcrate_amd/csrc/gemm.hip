@@ -480,7 +480,7 @@ int matmul_typed(uint32_t transposed, bool accumulate, uint64_t m, uint64_t k, u
                                               s, &done);
             if (done) return status;
         }
-        if (!in_place || small) {
+        if ((!in_place || small) && sliced_fits(m32, n32)) {
             if (a_kc && b_kc) {
                 launch_sliced<S, O, true, true>(pa, pb, pc, m32, k32, n32, accumulate, s);
             } else if (a_kc) {
@@ -490,24 +490,26 @@ int matmul_typed(uint32_t transposed, bool accumulate, uint64_t m, uint64_t k, u
             }
             return check_launch("matmul");
         }
-        if constexpr (std::is_same<S, float>::value) {
-            if (a_kc && b_kc) {
-                launch_inplace32<O, true, true>(pa, pb, pc, m32, k32, n32, accumulate, s);
-            } else if (a_kc) {
-                launch_inplace32<O, true, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
+        if (in_place) {
+            if constexpr (std::is_same<S, float>::value) {
+                if (a_kc && b_kc) {
+                    launch_inplace32<O, true, true>(pa, pb, pc, m32, k32, n32, accumulate, s);
+                } else if (a_kc) {
+                    launch_inplace32<O, true, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
+                } else {
+                    launch_inplace32<O, false, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
+                }
             } else {
-                launch_inplace32<O, false, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
+                if (a_kc && b_kc) {
+                    launch_tiled16<S, O, true, true>(pa, pb, pc, m32, k32, n32, accumulate, s);
+                } else if (a_kc) {
+                    launch_tiled16<S, O, true, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
+                } else {
+                    launch_tiled16<S, O, false, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
+                }
             }
-        } else {
-            if (a_kc && b_kc) {
-                launch_tiled16<S, O, true, true>(pa, pb, pc, m32, k32, n32, accumulate, s);
-            } else if (a_kc) {
-                launch_tiled16<S, O, true, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
-            } else {
-                launch_tiled16<S, O, false, false>(pa, pb, pc, m32, k32, n32, accumulate, s);
-            }
+            return check_launch("matmul");
         }
-        return check_launch("matmul");
     }
     void* made_a = nullptr;
     void* made_b = nullptr;

@@ -48,6 +48,13 @@ inline bool sliced_reach(uint64_t m, uint64_t k, uint64_t n, size_t width) {
     return m * k * width < limit && k * n * width < limit;
 }
 
+// Whether its grid is one a dispatch can hold, fewer than 2^32 work-items: 16 x 16
+// tiles of 512 threads pass that from 2^23 tiles on (16-bit 2^27 x 8 x 3).
+inline bool sliced_fits(uint32_t m, uint32_t n) {
+    const uint64_t tile = sliced_tile(m, n), threads = tile == 16 ? 512 : 256;
+    return ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * threads <= UINT32_MAX;
+}
+
 // Whether an f32 product takes 128 x 64 tiles rather than 128 x 128: where that
 // leaves fewer CUs waiting for the last of them.  A CU's time is its tiles' (two
 // at once share its matrix cores), and a narrow tile takes a little over half a
