@@ -79,6 +79,17 @@ def check(kind, out_kind, form, m, k, n, large_a):
     lib.call("tc_empty_cache")
 
 
+@pytest.mark.parametrize("form", [lib.PLAIN, lib.LEFT, lib.RIGHT], ids=["plain", "left", "right"])
+@pytest.mark.parametrize("kind,out_kind", [(lib.F32, lib.F32), (lib.BF16, lib.BF16), (lib.BF16, lib.F32),
+                                           (lib.F16, lib.F16), (lib.F16, lib.F32)],
+                         ids=["f32", "bf16", "bf16-f32", "f16", "f16-f32"])
+@pytest.mark.parametrize("large_a", [True, False], ids=["a", "b"])
+@pytest.mark.parametrize("k", [1032, 1029], ids=["words", "odd"])
+def test_operands_past_2_to_31_bytes(kind, out_kind, form, large_a, k):
+    many = (1 << 31) // (k * HOST[kind](0).itemsize) + 301
+    check(kind, out_kind, form, many if large_a else 21, k, 21 if large_a else many, large_a)
+
+
 @pytest.mark.parametrize("form", [lib.PLAIN, lib.LEFT], ids=["plain", "left"])
 @pytest.mark.parametrize("kind", [lib.BF16, lib.F16], ids=["bf16", "f16"])
 def test_more_small_tiles_than_a_dispatch_holds(kind, form):
