@@ -435,9 +435,11 @@ int launch_strided_binary(const S* a, const S* b, S* out, const Walk<3>& walk, u
     w.step_b = step_of(walk.strides[1][last]);
     const uint64_t run = walk.shape[last];
     constexpr int V = Pack<S>::N;
-    // Runs shorter than two words, or of elements apart on both sides, take an
-    // element a thread.
-    const bool words = run >= 2 * V && (w.step_a == kUnit || w.step_b == kUnit || run % V == 0);
+    // Whole words, and runs of over two with a side in order; shorter runs, and
+    // elements apart on both sides, take an element a thread.  A run of exactly
+    // one word is a word (us a call, an element a thread / a word: f32
+    // [20000000, 4] + [1, 4] 213 / 103, bf16 [10000000, 8] + [1, 8] 195 / 58).
+    const bool words = run % V == 0 || (run >= 2 * V && (w.step_a == kUnit || w.step_b == kUnit));
     const uint64_t run_groups = words ? (run + V - 1) / V : run;
     const uint64_t groups = count / run * run_groups;
     Div<I> per_run;
