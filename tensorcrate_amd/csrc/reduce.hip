@@ -29,6 +29,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <mutex>
 #include <unordered_map>
 
@@ -425,6 +426,7 @@ __global__ void __launch_bounds__(256) rows_kernel(const S* __restrict__ in, O* 
 template <typename I>
 struct ColumnWalk {
     Kept<I> outer;  // the kept axes before the column axis
+    I outers;       // their indexes
     I columns;
     I depth, step;
     I tiles;        // column tiles per outer index
@@ -432,9 +434,10 @@ struct ColumnWalk {
     I splits;       // depth splits across blocks
     I per_split;    // rows per split (the last may hold fewer)
     uint32_t lanes;   // lanes across a tile's columns
-    uint32_t groups;  // row groups: lanes x groups is at most a block's 256
+    uint32_t groups;  // row groups of one outer index
+    uint32_t held;    // outer indexes a block takes: lanes x groups x held is at most its 256
     bool apart;       // a group's rows are `groups` apart rather than a run of them
-    DivMod lanes_div;
+    DivMod lanes_div, groups_div;
 };
 
 // VC neighbouring columns of one row, 16 bytes of them or 4, wherever they start.
@@ -448,12 +451,13 @@ __device__ __forceinline__ void load_columns(const S* at, S (&v)[VC]) {
     }
 }
 
-// The states of a block's groups merged into group 0's, in a fixed order:
-// thread group * lanes + lane holds VC states.  Up to four groups meet at once;
-// more (narrow rows) first halve, a pair a step.
+// The states of each outer index's groups merged into its group 0's, in a fixed
+// order: thread (outer * groups + group) * lanes + lane holds VC states.  Up to
+// four groups meet at once; more (narrow rows) first halve, a pair a step.
 template <typename P, int VC>
 __device__ __forceinline__ void merge_groups(typename P::State (&s)[VC], typename P::State (*stage)[256],
                                              uint32_t group, uint32_t groups, uint32_t lanes) {
+    if (groups == 1) return;
     while (groups > 4) {
         const uint32_t half = (groups + 1) / 2;
         if (group >= half) {
@@ -484,15 +488,19 @@ __device__ __forceinline__ void merge_groups(typename P::State (&s)[VC], typenam
 
 // One block: `lanes` lanes on VC neighbouring columns each (one word, wherever
 // it starts; a last word that would pass the columns starts earlier and its
-// first columns are not written; at least VC columns), times
-// `groups` row groups sharing one split's rows, eight rows in flight a lane.
-// With splits == 1 it finishes the results; otherwise it writes its states to
-// `partial[result * splits + split]` for the combine kernels.
+// first columns are not written; at least VC columns), times `groups` row groups
+// sharing one split's rows, eight rows in flight a lane, times `held` outer
+// indexes.  With splits == 1 it finishes the results; otherwise it writes its
+// states to `partial[result * splits + split]` for the combine kernels.
 // Bound by loads in flight and by how evenly the columns fill the lanes.  WIDE:
 // 64 lanes, four groups, each a run of rows.  us a call with its launches,
 // before (64 lanes, one column each; under 16 columns a thread a result) /
 // this: bf16 [60480 x 11] sums 7877 / 6.3, [11550 x 513] 9.5 / 8.6; f32
-// [14688 x 11] 1700 / 6.3, [8192 x 1024] 9.0 / 9.0.
+// [14688 x 11] 1700 / 6.3, [8192 x 1024] 9.0 / 9.0.  Over many outer indexes a
+// block each leaves most of it idle, and a chip takes some 0.6 ns a block: f32
+// [1000000, 4, 2] sums over axis 1, a thread a result / a block an outer index /
+// this, 14.1 / 613 / 13.2; [250000, 32, 8] 77 / 243 / 39; [60606, 32, 33] 84 / 63 /
+// 38.
 template <typename S, typename P, typename O, int VC, bool WIDE, bool NT, typename I>
 __global__ void __launch_bounds__(256) columns_kernel(const S* __restrict__ in, O* __restrict__ out,
                                                       typename P::State* __restrict__ partial,
@@ -503,16 +511,20 @@ __global__ void __launch_bounds__(256) columns_kernel(const S* __restrict__ in, 
     __shared__ State stage[VC][256];
     const uint32_t lanes = WIDE ? 64 : w.lanes, groups = WIDE ? 4 : w.groups;
     const bool apart = !WIDE && w.apart;
-    const uint32_t group = WIDE ? threadIdx.x / 64 : w.lanes_div.div(threadIdx.x);
-    const uint32_t lane = threadIdx.x - group * lanes;
+    const uint32_t across = WIDE ? threadIdx.x / 64 : w.lanes_div.div(threadIdx.x);
+    const uint32_t lane = threadIdx.x - across * lanes;
+    const uint32_t within = WIDE ? 0 : w.groups_div.div(across);
+    // Past the block's outer indexes: a group that takes no rows.
+    const uint32_t group = !WIDE && within >= w.held ? groups : across - within * groups;
     for (I block = blockIdx.x; block < blocks; block += gridDim.x) {
-        // block -> (split, outer, tile), split outermost so neighbouring
+        // block -> (split, outers, tile), split outermost so neighbouring
         // blocks share rows.
         const I per_split_blocks = blocks / w.splits;
         const I split = block / per_split_blocks;
         const I rest = block - split * per_split_blocks;
-        const I outer = w.tiles_div.div(rest);
-        const I tile = rest - outer * w.tiles;
+        const I first = w.tiles_div.div(rest);
+        const I tile = rest - first * w.tiles;
+        const I outer = WIDE ? first : first * w.held + within;
         const I column = (tile * lanes + lane) * VC;
         const I from = VC > 1 && column + VC > w.columns ? w.columns - VC : column;
         const I row_begin = split * w.per_split;
@@ -521,7 +533,8 @@ __global__ void __launch_bounds__(256) columns_kernel(const S* __restrict__ in, 
         State s[VC];
 #pragma unroll
         for (int c = 0; c < VC; c++) s[c] = P::init();
-        if (column < w.columns && group < groups) {
+        const bool live = column < w.columns && outer < w.outers;
+        if (live && group < groups) {
             const S* base = in + kept_offset(w.outer, outer) + from;
             const I hop = apart ? groups : 1;
             const I run = apart ? 1 : (row_end - row_begin + groups - 1) / groups;
@@ -543,20 +556,29 @@ __global__ void __launch_bounds__(256) columns_kernel(const S* __restrict__ in, 
             }
             if (row < end) {
                 const uint32_t left = static_cast<uint32_t>((end - row + hop - 1) / hop);
-                S v[U][VC];
+                auto add_rest = [&](auto most) __attribute__((always_inline)) {
+                    constexpr int R = decltype(most)::value;
+                    S v[R][VC];
 #pragma unroll
-                for (int k = 0; k < U; k++) load_columns<NT>(at + (k < left ? k : 0) * next, v[k]);
+                    for (int k = 0; k < R; k++) load_columns<NT>(at + (k < left ? k : 0) * next, v[k]);
 #pragma unroll
-                for (int c = 0; c < VC; c++) {
-                    float x[U];
+                    for (int c = 0; c < VC; c++) {
+                        float x[R];
 #pragma unroll
-                    for (int k = 0; k < U; k++) x[k] = E::widen(v[k][c]);
-                    P::template add_some<U, 1>(s[c], x, left, static_cast<uint32_t>(row), static_cast<uint32_t>(hop));
+                        for (int k = 0; k < R; k++) x[k] = E::widen(v[k][c]);
+                        P::template add_some<R, 1>(s[c], x, left, static_cast<uint32_t>(row),
+                                                   static_cast<uint32_t>(hop));
+                    }
+                };
+                if (!WIDE && left <= U / 2) {
+                    add_rest(std::integral_constant<int, U / 2>{});
+                } else {
+                    add_rest(std::integral_constant<int, U>{});
                 }
             }
         }
         merge_groups<P, VC>(s, stage, group, groups, lanes);
-        if (group == 0 && column < w.columns) {
+        if (live && group == 0) {
 #pragma unroll
             for (int c = 0; c < VC; c++) {
                 if (from + c < column) continue;
@@ -721,21 +743,41 @@ int launch_columns(const S* in, O* out, const Plan& plan, const Finish& f, hipSt
     // Tiles of 64 lanes, or evenly narrower ones where those would leave over
     // a seventh of the lanes without columns (the constant shape runs a sixth
     // faster: bf16 [500, 200, 1000] argmax over axis 1, 66 us in tiles of 63
-    // lanes, 56 in 64), the rest of the block on other rows.  Four blocks a CU: what the tiles leave missing is made up by
-    // splitting the depth, each group keeping four rounds of eight rows, since
-    // a split costs a second kernel (2.5 us) and a state a result.
+    // lanes, 56 in 64).  The rest of the block takes other rows, and other outer
+    // indexes where the rows are few.  Four blocks a CU: what the tiles leave
+    // missing is made up by splitting the depth, each group keeping four rounds
+    // of eight rows, since a split costs a second kernel (2.5 us) and a state a
+    // result.
     const uint64_t want = static_cast<uint64_t>(compute_units()) * 4;
     uint64_t tiles = (words + 63) / 64;
     const uint64_t lanes = words * 8 >= tiles * 64 * 7 ? 64 : (words + tiles - 1) / tiles;
     tiles = (words + lanes - 1) / lanes;
-    const uint64_t groups = std::min<uint64_t>(256 / lanes, depth);
-    const uint64_t base_blocks = outer * tiles;
+    // Rows of under 64 bytes: neighbouring groups on neighbouring rows share
+    // their lines.  Wider ones: a run of rows a group, since rows a power of
+    // two apart are apt to share a memory channel (f32 [65536 x 2048] sums:
+    // 98 us apart, 82 in runs).
+    const bool apart = lanes * VC * sizeof(S) < 64;
+    // A round of eight rows a group or more.  Groups cost a merge, so wider rows
+    // take no more than fill those blocks, in whole rounds (f32 [60606, 32, 33]
+    // sums, four groups / one: 44 / 38 us); the four groups of 64 lanes stay, for
+    // the constant shape (bf16 [7812, 128, 256] argmax, one group / four: 17.3 /
+    // 12.7).
+    const uint64_t slots = 256 / lanes;
+    uint64_t groups = std::min(slots, (depth + 7) / 8);
+    if (!apart && (lanes < 64 || groups < 4)) {
+        groups = std::max<uint64_t>(1, std::min(groups, want * 256 / (outer * tiles * lanes)));
+        const uint64_t run = (depth + 8 * groups - 1) / (8 * groups) * 8;
+        groups = (depth + run - 1) / run;
+    }
+    const uint64_t held = std::min(slots / groups, outer);
+    const uint64_t base_blocks = (outer + held - 1) / held * tiles;
     uint64_t splits = 1;
     if (base_blocks * 2 <= want) {
         splits = std::min((want + base_blocks - 1) / base_blocks, depth / (groups * 32));
     }
     const Cut<typename P::State> cut(depth, splits, 1, results);
     splits = cut.splits;
+    w.outers = static_cast<I>(outer);
     w.columns = static_cast<I>(columns);
     w.depth = static_cast<I>(depth);
     w.step = static_cast<I>(plan.folded.strides[0]);
@@ -745,19 +787,18 @@ int launch_columns(const S* in, O* out, const Plan& plan, const Finish& f, hipSt
     w.per_split = static_cast<I>(cut.per_split);
     w.lanes = static_cast<uint32_t>(lanes);
     w.groups = static_cast<uint32_t>(groups);
-    // Rows of under 64 bytes: neighbouring groups on neighbouring rows share
-    // their lines.  Wider ones: a run of rows a group, since rows a power of
-    // two apart are apt to share a memory channel (f32 [65536 x 2048] sums:
-    // 98 us apart, 82 in runs).
-    w.apart = lanes * VC * sizeof(S) < 64;
+    w.held = static_cast<uint32_t>(held);
+    w.apart = apart;
     w.lanes_div = DivMod(w.lanes);
+    w.groups_div = DivMod(w.groups);
     const uint64_t blocks = base_blocks * splits;
     typename P::State* partial = cut.partial;
-    const uint32_t grid = grid_for(blocks, 1, 64);
+    const uint32_t grid = grid_for(blocks, 1, 64), threads = static_cast<uint32_t>(lanes * groups * held + 63) / 64 * 64;
     if (lanes == 64 && groups == 4) {
         columns_kernel<S, P, O, VC, true, NT, I><<<grid, 256, 0, s>>>(in, out, partial, w, static_cast<I>(blocks), f);
     } else {
-        columns_kernel<S, P, O, VC, false, NT, I><<<grid, 256, 0, s>>>(in, out, partial, w, static_cast<I>(blocks), f);
+        columns_kernel<S, P, O, VC, false, NT, I><<<grid, threads, 0, s>>>(in, out, partial, w, static_cast<I>(blocks),
+                                                                           f);
     }
     int status = check_launch(what);
     if (status == TC_OK && splits > 1) status = launch_combine<P, O, I>(partial, out, results, splits, f, s, what);
@@ -816,9 +857,11 @@ int launch_reduce(const S* in, O* out, const Plan& plan, const Finish& f, hipStr
         if (stream) return launch_rows<S, P, O, true, I>(in, out, plan, f, s, what);
         return launch_rows<S, P, O, false, I>(in, out, plan, f, s, what);
     }
-    // Columns: contiguous neighbouring results, one strided folded axis, not
-    // empty (there is nothing to spread: the general kernel answers).
-    if (depth > 0 && folded.rank == 1 && kept.rank >= 1 && kept.strides[kept.rank - 1] == 1) {
+    // Columns: contiguous neighbouring results, one strided folded axis of more
+    // than the one or two rows that leave nothing to spread or keep in flight
+    // (two rows, 2000000 results in f32: 12 us with any columns, 10 in the
+    // general kernel; four 13 and 14).
+    if (depth > 2 && folded.rank == 1 && kept.rank >= 1 && kept.strides[kept.rank - 1] == 1) {
         // An input past the Infinity Cache streams with 16-byte words.  A
         // smaller one takes 4 bytes of columns a lane, which spreads it over
         // four times the threads, and one column for variances and

@@ -47,3 +47,26 @@ def test_broadcasts_over_runs_of_one_word(kind, run):
     # An element a thread where the run was one word: 2.0 (f32), 3.3 (16-bit).
     rows = 10_000_000
     assert ratio(broadcast_add(kind, rows, run), broadcast_add(kind, rows // 2, run * 2), 4) < 1.5
+
+
+def reduction(kind, op, shape, axis):
+    """The maximum or its index along `axis`, into the leading part of `out`."""
+    n, size = int(np.prod(shape)), lib.DTYPE_SIZE[kind]
+    source, out = lib.Buffer(n * size), lib.Buffer(n // shape[axis] * 4)
+    zero = np.zeros(1, lib.NUMPY_TYPE[kind])
+    lib.call("tc_fill", source.ptr, n, size, zero.ctypes.data)
+    steps = [int(np.prod(shape[k + 1:])) for k in range(len(shape))]
+    kept = [k for k in range(len(shape)) if k != axis]
+    split = lib.split(0, [shape[k] for k in kept], [steps[k] for k in kept], [shape[axis]], [steps[axis]])
+    if op == "argmax":
+        return lambda: lib.call("tc_arg_reduce", kind, source.ptr, n, ctypes.byref(split), lib.RMAX, out.ptr)
+    return lambda: lib.call("tc_reduce_axes", kind, source.ptr, n, ctypes.byref(split), lib.FOLD, lib.SUM, 0, out.ptr)
+
+
+@pytest.mark.parametrize("op", ["sum", "argmax"])
+@pytest.mark.parametrize("columns,outers", [(2, 500_000), (8, 100_000), (15, 50_000)])
+def test_narrow_columns_under_many_outer_indexes(op, columns, outers):
+    # Half the elements in sixteen times the outer indexes, against a depth of
+    # 64: a block an outer index took 4.7 to 5 times as long (2 columns), 3.1 to 3.7.
+    first, second = (outers, 4, columns), (outers // 8, 64, columns)
+    assert ratio(reduction(lib.F32, op, first, 1), reduction(lib.F32, op, second, 1), 20) < 1.5

@@ -1,8 +1,8 @@
 """The reduction kernels' lane and row splits at the sizes where they change:
 a few lanes a slice, a whole wave, a slice cut over blocks; columns narrower
 than a word, narrower than a tile, tiles of 64 and of fewer lanes, runs of rows
-and rows apart, a depth split over blocks; and all of them starting off 16
-bytes.  Extremes and arg-reductions are exact, with NaNs, infinities and ties
+and rows apart, several outer indexes a block, a depth split over blocks; and all
+of them starting off 16 bytes.  Extremes and arg-reductions are exact, with NaNs, infinities and ties
 among the values; sums, means and variances are within the bound of
 tests/test_gpu_reduce.py of f64."""
 
@@ -26,6 +26,11 @@ ROWS += [([700, 37], [1]), ([3, 40, 61], [2]), ([1, 70001], [1]), ([3, 50011], [
 # Columns: narrower than any word, odd, a tile, tiles, with outer axes; depths
 # within a group, of a few rounds, and split.
 COLUMNS = [([d, c], [0]) for d in (2, 5, 33, 700) for c in (2, 3, 5, 8, 11, 16, 31, 64, 65, 257)]
+COLUMNS += [([d, c], [0]) for d in (3, 4, 9, 17) for c in (3, 16, 33, 64)]
+# Several outer indexes a block, and a last block of fewer: one group each and
+# more, narrow rows and wide, with one column a lane and with words.
+COLUMNS += [([o, d, c], [1]) for o, d, c in [(301, 3, 2), (301, 8, 3), (130, 33, 7), (97, 70, 5), (3000, 20, 10),
+                                             (701, 6, 33), (2500, 50, 33), (53, 9, 64), (40, 17, 100), (9, 30, 130)]]
 COLUMNS += [([9000, c], [0]) for c in (2, 7, 11, 40, 130)] + [([6, 77, 57], [1]), ([3, 300, 9], [1]), ([40, 9, 130], [0, 1])]
 CASES = ROWS + COLUMNS
 
