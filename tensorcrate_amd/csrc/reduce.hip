@@ -391,18 +391,30 @@ __global__ void __launch_bounds__(256) rows_kernel(const S* __restrict__ in, O* 
             }
             const S* slice = in + kept_offset(w.kept, result) + begin;
             const I packs = count / V;
+            // Whole rounds for all of the slice's lanes, then the rest for all
+            // of them, so that no lane runs one part while another waits.
+            const I rounds = packs / (lanes * U);
             I p = at;
-            for (; p + lanes * (U - 1) < packs; p += lanes * U) {
+            for (I k = 0; k < rounds; k++, p += lanes * U) {
                 float x[U * V];
                 load_packs<S, U, NT, false, I>(slice, p, lanes, 0, x);
                 P::template add_packs<U, V>(s, x, static_cast<uint32_t>(begin + p * V), static_cast<uint32_t>(lanes * V));
             }
-            if (p < packs) {
-                float x[U * V];
-                load_packs<S, U, NT, true, I>(slice, p, lanes, packs - 1, x);
+            auto add_rest = [&](auto most) __attribute__((always_inline)) {
+                constexpr int R = decltype(most)::value;
+                if (p >= packs) return;
+                float x[R * V];
+                load_packs<S, R, NT, true, I>(slice, p, lanes, packs - 1, x);
                 const uint32_t left = static_cast<uint32_t>((packs - p + lanes - 1) / lanes);
-                P::template add_some<U, V>(s, x, left, static_cast<uint32_t>(begin + p * V),
+                P::template add_some<R, V>(s, x, left, static_cast<uint32_t>(begin + p * V),
                                            static_cast<uint32_t>(lanes * V));
+            };
+            if (!P::kLight && packs - rounds * lanes * U <= lanes) {
+                add_rest(std::integral_constant<int, 1>{});
+            } else if (!P::kLight && packs - rounds * lanes * U <= lanes * 2) {
+                add_rest(std::integral_constant<int, 2>{});
+            } else {
+                add_rest(std::integral_constant<int, U>{});
             }
             for (I i = packs * V + at; i < count; i += lanes) {
                 P::add(s, E::widen(slice[i]), static_cast<uint32_t>(begin + i));
@@ -816,11 +828,18 @@ int launch_rows(const S* in, O* out, const Plan& plan, const Finish& f, hipStrea
     w.kept = make_kept<I>(plan.kept, plan.kept.rank);
     w.results = static_cast<I>(results);
     w.depth = static_cast<I>(depth);
+    // Variances and arg-reductions are bound by their arithmetic, so they take a
+    // quarter as many lanes as packs only where the rows then still make four
+    // blocks a CU, and otherwise a lane a pack (bf16 argmax, a quarter / a lane:
+    // [1000, 1000] 8.4 / 4.2 us, [1000, 400] 6.0 / 3.7).
+    const uint64_t want = static_cast<uint64_t>(compute_units()) * 4, round = 64 * V * 4;
     uint64_t lanes = 64;
-    while (lanes > 1 && depth / V < lanes * 4) lanes /= 2;
+    while (lanes > 1 && (depth / V <= lanes / 2 ||
+                         (depth / V < lanes * 4 && (P::kLight || results * lanes > want * 256)))) {
+        lanes /= 2;
+    }
     // A few long slices: cut until there are four waves a CU, each cut eight
     // rounds of a wave's loads or more.
-    const uint64_t want = static_cast<uint64_t>(compute_units()) * 4, round = 64 * V * 4;
     uint64_t splits = 1;
     if (lanes == 64 && results < want) splits = std::min((want + results - 1) / results, depth / (round * 8));
     const Cut<typename P::State> cut(depth, splits, V, results);

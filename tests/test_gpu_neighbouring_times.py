@@ -66,7 +66,14 @@ def reduction(kind, op, shape, axis):
 @pytest.mark.parametrize("op", ["sum", "argmax"])
 @pytest.mark.parametrize("columns,outers", [(2, 500_000), (8, 100_000), (15, 50_000)])
 def test_narrow_columns_under_many_outer_indexes(op, columns, outers):
-    # Half the elements in sixteen times the outer indexes, against a depth of
+    # Half the elements in eight times the outer indexes, against a depth of
     # 64: a block an outer index took 4.7 to 5 times as long (2 columns), 3.1 to 3.7.
     first, second = (outers, 4, columns), (outers // 8, 64, columns)
     assert ratio(reduction(lib.F32, op, first, 1), reduction(lib.F32, op, second, 1), 20) < 1.5
+
+
+@pytest.mark.parametrize("rows", [300, 3000])
+def test_arg_reductions_of_a_part_round_of_words(rows):
+    # 125 words a row against 128: 1.6 and 1.8 times as long where a row took
+    # few lanes and they left its last whole round at different words.
+    assert ratio(reduction(lib.BF16, "argmax", (rows, 1000), 1), reduction(lib.BF16, "argmax", (rows, 1024), 1), 100) < 1.3

@@ -22,6 +22,9 @@ pytestmark = pytest.mark.gpu
 # (shape, folded axes).  Rows: every count of lanes from one to 64, with and
 # without a part word, whole groups of words and parts of them.
 ROWS = [([5, n], [1]) for n in (2, 3, 4, 7, 8, 9, 15, 16, 33, 63, 64, 65, 127, 130, 255, 513, 1023, 1024, 2049, 5000)]
+# Enough rows that variances and arg-reductions take few lanes a row too; 125
+# words of 16-bit elements are a whole round of some lanes only.
+ROWS += [([9000, n], [1]) for n in (100, 257, 1000)]
 ROWS += [([700, 37], [1]), ([3, 40, 61], [2]), ([1, 70001], [1]), ([3, 50011], [1]), ([2, 3, 30001], [1, 2])]
 # Columns: narrower than any word, odd, a tile, tiles, with outer axes; depths
 # within a group, of a few rounds, and split.
