@@ -541,15 +541,18 @@ bool compile_program(const std::string& source, const std::vector<std::string>& 
     return true;
 }
 
-// The cached kernels of `source` for this device, compiled on the source's
-// second request; false (run something else) before that or if it does not
-// compile.
+// The cached `kernels` of `source` for this device, compiled on their second
+// request; false (run something else) before that or if it does not compile.
+// A source alone does not say which kernels: a product's epilogue is written
+// for a group of elements, whatever the kernel's type, tile and waves.
 bool cached_kernels(const std::string& source, const std::vector<std::string>& kernels, hipFunction_t* out,
                     KernelResources* resources = nullptr) {
     int device = 0;
     (void)hipGetDevice(&device);
     std::lock_guard<std::mutex> lock(compiled_mutex);
-    Compiled& entry = compiled_programs["device " + std::to_string(device) + "\n" + source];
+    std::string key = "device " + std::to_string(device) + "\n";
+    for (const std::string& kernel : kernels) key += kernel + "\n";
+    Compiled& entry = compiled_programs[key + source];
     if (entry.failed) return false;
     if (entry.functions.empty()) {
         if (++entry.seen < 2) return false;

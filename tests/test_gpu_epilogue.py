@@ -111,6 +111,21 @@ def test_the_product_must_be_read_in_order():
                             [(lib.Buffer.of(np.ones(n, np.float32)), n)], [(out, m * n)])
 
 
+def test_programs_that_name_no_type_are_compiled_for_each():
+    # A constant stored in f32: its source is the same for every product type,
+    # and each has kernels of its own.
+    m, k, n = 1928, 200, 1992
+    code = Code()
+    code.store(code.const(1.5), lib.F32, 0)
+    for kind in (lib.BF16, lib.F32, lib.F16):
+        a, w = (lib.Buffer.of(np.zeros(shape, HOST[kind])) for shape in ((m, k), (k, n)))
+        for _ in range(3):
+            out = lib.Buffer(m * n * 4)
+            lib.call("tc_fill", out.ptr, m * n, 4, np.zeros(1, np.float32).ctypes.data)
+            lib.matmul_epilogue(kind, code.code, [identity_place(m, n)], a, w, m, k, n, [], [(out, m * n)])
+            assert np.all(out.download(np.float32, m * n) == 1.5)
+
+
 @pytest.mark.parametrize("kind", [lib.F32, lib.BF16, lib.F16])
 @pytest.mark.parametrize("m,k,n", [(520, 136, 1032), (4100, 136, 4104), (4100, 200, 4104), (4100, 256, 4104)],
                          ids=["small-tiles", "large-tiles", "persistent", "four-wave"])
