@@ -586,8 +586,12 @@ bool run_compiled_sliced(uint32_t dtype, uint32_t m, uint32_t k, uint32_t n, con
                          uint32_t input_count, void* const* outputs, uint32_t output_count, hipStream_t s,
                          int* status) {
     const uint32_t tile = sliced_tile(m, n);
+    const bool two = sliced_waves(m, k, n, dtype == TC_F32 ? 4 : 2) == 2;
     const std::string type = dtype == TC_F32 ? "float" : dtype == TC_F16 ? "_Float16" : "tc::bf16_t";
-    const std::string shape = tile == 64 ? "4, 4, 4, 1" : tile == 32 ? "2, 2, 4, 1" : "1, 1, 8, 4";
+    const std::string shape = tile == 64   ? "4, 4, 4, 1"
+                              : tile == 32 ? "2, 2, 4, 1"
+                              : two        ? "1, 1, 2, 1"
+                                           : "1, 1, 8, 4";
     std::vector<float> constants;
     const std::string source = epilogue_source(dtype, code, count, host_places, &constants, false, nullptr,
                                                static_cast<int>(tile / 4), "gemm_sliced.hpp");
@@ -603,9 +607,9 @@ bool run_compiled_sliced(uint32_t dtype, uint32_t m, uint32_t k, uint32_t n, con
     bool accumulate = false;
     void* params[] = {const_cast<void**>(&a), const_cast<void**>(&b), &none, &m, &n, &k, &accumulate, &args};
     const uint32_t blocks = ((m + tile - 1) / tile) * ((n + tile - 1) / tile);
+    const uint32_t threads = tile != 16 ? 256 : two ? 128 : 512;
     count_dispatch();
-    const hipError_t error =
-        hipModuleLaunchKernel(function, blocks, 1, 1, tile == 16 ? 512 : 256, 1, 1, 0, s, params, nullptr);
+    const hipError_t error = hipModuleLaunchKernel(function, blocks, 1, 1, threads, 1, 1, 0, s, params, nullptr);
     *status = error == hipSuccess ? TC_OK : fail(TC_DEVICE, std::string("fused matmul: ") + hipGetErrorString(error));
     return true;
 }

@@ -48,6 +48,15 @@ inline bool sliced_reach(uint64_t m, uint64_t k, uint64_t n, size_t width) {
     return m * k * width < limit && k * n * width < limit;
 }
 
+// The waves that share a 16 x 16 tile's K: eight, or two where four chunks are all
+// of K and there are more tiles than blocks of eight waves are resident, which
+// then wait for one another (us a call, eight / two: f32 1000000 x 8 x 16 173 /
+// 42, 1000000 x 32 x 16 143 / 31, bf16 1000000 x 16 x 10 157 / 41).
+inline uint32_t sliced_waves(uint32_t m, uint32_t k, uint32_t n, size_t width) {
+    const uint64_t tiles = static_cast<uint64_t>((m + 15) / 16) * ((n + 15) / 16);
+    return k * width <= 256 && tiles > static_cast<uint64_t>(compute_units()) * 4 ? 2 : 8;
+}
+
 // Whether its grid is one a dispatch can hold, fewer than 2^32 work-items: 16 x 16
 // tiles of 512 threads pass that from 2^23 tiles on (16-bit 2^27 x 8 x 3).
 inline bool sliced_fits(uint32_t m, uint32_t n) {
@@ -160,6 +169,8 @@ void launch_sliced(const S* a, const S* b, O* c, uint32_t m, uint32_t k, uint32_
         sliced_kernel<S, O, A_KC, B_KC, 4, 4, 4, 1, EPI><<<blocks, 256, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
     } else if (tile == 32) {
         sliced_kernel<S, O, A_KC, B_KC, 2, 2, 4, 1, EPI><<<blocks, 256, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
+    } else if (sliced_waves(m, k, n, sizeof(S)) == 2) {
+        sliced_kernel<S, O, A_KC, B_KC, 1, 1, 2, 1, EPI><<<blocks, 128, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
     } else {
         sliced_kernel<S, O, A_KC, B_KC, 1, 1, 8, 4, EPI><<<blocks, 512, 0, s>>>(a, b, c, m, n, k, accumulate, epi);
     }

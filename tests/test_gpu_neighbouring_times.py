@@ -77,3 +77,19 @@ def test_arg_reductions_of_a_part_round_of_words(rows):
     # 125 words a row against 128: 1.6 and 1.8 times as long where a row took
     # few lanes and they left its last whole round at different words.
     assert ratio(reduction(lib.BF16, "argmax", (rows, 1000), 1), reduction(lib.BF16, "argmax", (rows, 1024), 1), 100) < 1.3
+
+
+def product(kind, m, k, n):
+    size = lib.DTYPE_SIZE[kind]
+    a, b, c = lib.Buffer(m * k * size), lib.Buffer(k * n * size), lib.Buffer(m * n * size)
+    for x, count in ((a, m * k), (b, k * n)):
+        zero = np.zeros(1, lib.NUMPY_TYPE[kind])
+        lib.call("tc_fill", x.ptr, count, size, zero.ctypes.data)
+    return lambda: lib.call("tc_matmul", kind, kind, lib.PLAIN, 0, m, k, n, a.ptr, b.ptr, c.ptr)
+
+
+@pytest.mark.parametrize("kind,k,n", [(lib.F32, 8, 16), (lib.F32, 32, 16), (lib.BF16, 16, 10)])
+def test_products_of_few_columns_over_a_short_k(kind, k, n):
+    # 16 x 16 tiles of eight waves, most of them with no K to read: 9 to 10 us
+    # of them wait for one another.
+    assert ratio(product(kind, 1_000_000, k, n), product(kind, 1_000_000, k, 64), 3) < 1.0

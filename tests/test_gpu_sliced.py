@@ -25,6 +25,9 @@ IDS = {lib.F32: "f32", lib.F16: "f16", lib.BF16: "bf16"}
 SHAPES = [(2, 8, 2), (16, 8, 16), (17, 31, 15), (15, 32, 33), (40, 33, 24), (33, 127, 65), (16, 1024, 48),
           (31, 1057, 16), (64, 2085, 50), (512, 96, 256), (500, 70, 301), (33, 64, 4000), (511, 4097, 263),
           (1024, 64, 512), (1000, 130, 601), (35, 77, 8200), (2048, 40, 2047), (9000, 24, 3), (2, 17, 5000)]
+# Over 1024 tiles of 16 x 16, which two waves share up to K of 64 in 32 bits and of
+# 128 in 16: less than a chunk, whole chunks, the last such K and the next.
+SHAPES += [(17000, 8, 3), (16500, 64, 16), (16500, 65, 11), (10, 31, 17000), (16600, 128, 9), (16600, 129, 16)]
 
 
 def operands(kind, form, m, k, n, seed):
@@ -81,7 +84,8 @@ def test_operands_at_any_address_and_values_past_the_edges(kind, form):
 
 
 @pytest.mark.parametrize("kind", [lib.F32, lib.BF16, lib.F16], ids=IDS.get)
-@pytest.mark.parametrize("m,k,n", [(24, 40, 40), (264, 200, 512), (1000, 64, 520)], ids=["16", "32", "64"])
+@pytest.mark.parametrize("m,k,n", [(24, 40, 40), (264, 200, 512), (1000, 64, 520), (17000, 56, 16)],
+                         ids=["16", "32", "64", "16 of two waves"])
 def test_a_program_in_the_epilogue_gives_the_unfused_bits(kind, m, k, n):
     # Every tile's epilogue, interpreted on the first call and compiled from
     # the second, against the product and then the program.
