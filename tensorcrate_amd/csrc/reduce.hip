@@ -834,8 +834,9 @@ int launch_rows(const S* in, O* out, const Plan& plan, const Finish& f, hipStrea
     // [1000, 1000] 8.4 / 4.2 us, [1000, 400] 6.0 / 3.7).
     const uint64_t want = static_cast<uint64_t>(compute_units()) * 4, round = 64 * V * 4;
     uint64_t lanes = 64;
-    while (lanes > 1 && (depth / V <= lanes / 2 ||
-                         (depth / V < lanes * 4 && (P::kLight || results * lanes > want * 256)))) {
+    const uint64_t packs = depth / V;
+    while (lanes > 1 && (packs <= lanes / 2 ||
+                         (packs < lanes * 4 && (P::kLight || results * lanes >= want * 256)))) {
         lanes /= 2;
     }
     // A few long slices: cut until there are four waves a CU, each cut eight

@@ -90,6 +90,6 @@ def product(kind, m, k, n):
 
 @pytest.mark.parametrize("kind,k,n", [(lib.F32, 8, 16), (lib.F32, 32, 16), (lib.BF16, 16, 10)])
 def test_products_of_few_columns_over_a_short_k(kind, k, n):
-    # 16 x 16 tiles of eight waves, most of them with no K to read: 9 to 10 us
-    # of them wait for one another.
+    # 16 x 16 tiles of eight waves, most of them with no K to read, took 1.7, 1.4
+    # and 1.3 times as long as 64 columns, which write four times as much.
     assert ratio(product(kind, 1_000_000, k, n), product(kind, 1_000_000, k, 64), 3) < 1.0
