@@ -67,7 +67,10 @@ def run_both(kind, program, m, k, n, seed):
             [p.download(t, m * n) for p, t in zip(plain, dtypes)])
 
 
-SHAPES = [(8, 8, 8), (64, 64, 64), (300, 256, 520), (1024, 512, 1024), (4096, 64, 4096), (4100, 72, 4104)]
+# Small products (the register-fed kernel), ones of fewer 256 x 256 tiles than CUs,
+# and larger.
+SHAPES = [(8, 8, 8), (64, 64, 64), (300, 256, 520), (1024, 512, 1024), (2048, 136, 2056), (1928, 200, 1992),
+          (4096, 64, 4096), (4100, 72, 4104)]
 
 
 @pytest.mark.parametrize("kind", [lib.F32, lib.BF16, lib.F16])
@@ -127,19 +130,20 @@ def test_programs_that_name_no_type_are_compiled_for_each():
 
 
 @pytest.mark.parametrize("kind", [lib.F32, lib.BF16, lib.F16])
-@pytest.mark.parametrize("m,k,n", [(520, 136, 1032), (4100, 136, 4104), (4100, 200, 4104), (4100, 256, 4104)],
-                         ids=["small-tiles", "large-tiles", "persistent", "four-wave"])
+@pytest.mark.parametrize("m,k,n", [(520, 136, 1032), (1928, 136, 1992), (4100, 136, 4104), (4100, 200, 4104),
+                                   (4100, 256, 4104)],
+                         ids=["register-fed", "small-tiles", "large-tiles", "persistent", "four-wave"])
 def test_a_repeated_program_runs_compiled_with_the_same_bits(kind, m, k, n):
     # The first appearance of a program runs the interpreter epilogue; from
     # the second the program is compiled into the product kernel (as the
     # reference's Metal backend specializes a program seen before).  All
-    # give the unfused bits: in the kernel for fewer 256 x 256 tiles than
-    # CUs, in the one-tile kernel for more (17 x 17 tiles, ragged, three
+    # give the unfused bits: in the register-fed kernel for small products,
+    # in the kernel for fewer 256 x 256 tiles than CUs, in the one-tile kernel for more (17 x 17 tiles, ragged, three
     # steps), and, for 16-bit types with a whole pair of steps, in the
     # eight-wave persistent kernel, or with K a multiple of 128 in the
     # four-wave one.  Compiled kernels are cached by source, constants being
     # arguments, so each case has a program of its own shape: the bias added
-    # for the small tiles, subtracted for the large ones, the scaled
+    # for the register-fed one, multiplied for the small tiles, subtracted for the large ones, the scaled
     # product's maximum with the bias for the persistent ones, and the
     # minimum of product plus bias with a constant for the four-wave ones.
     code = Code()
@@ -152,7 +156,7 @@ def test_a_repeated_program_runs_compiled_with_the_same_bits(kind, m, k, n):
         scaled = code.binary(lib.MUL, p, code.const(0.375 + kind))
         code.store(code.compare(lib.MAX, scaled, b), kind, 0)
     else:
-        shifted = code.binary(lib.SUB if m > 1000 else lib.ADD, p, b)
+        shifted = code.binary({520: lib.ADD, 1928: lib.MUL}.get(m, lib.SUB), p, b)
         scaled = code.binary(lib.MUL, shifted, code.const(0.375 + kind))
         code.store(code.compare(lib.MAX, scaled, code.const(-0.25)), kind, 0)
     rng = np.random.default_rng(kind)

@@ -12,10 +12,10 @@ from tensorcrate_amd import lib
 pytestmark = pytest.mark.gpu
 
 # Operands of whole 16-byte rows, more than a 64 x 64 tile a compute unit (256):
-# one K step with most of it missing, then one, two, three and many, whole and
-# ragged; 128 x 64 tiles (the first six) and 128 x 128, with a last tile of one
-# row or of four columns, and whole.
-SHAPES = [(1152, 4, 1152), (1152, 32, 1152), (1028, 36, 1156), (1284, 64, 1028), (1156, 68, 1152), (1028, 1000, 1092),
+# one K step with most of it missing (K below 8 goes to another kernel), then one,
+# two, three and many, whole and ragged; 128 x 64 tiles (the first seven) and 128 x
+# 128, with a last tile of one row or of four columns, and whole.
+SHAPES = [(1152, 8, 1152), (1156, 12, 1028), (1152, 32, 1152), (1028, 36, 1156), (1284, 64, 1028), (1156, 68, 1152), (1028, 1000, 1092),
           (2048, 32, 2048), (2048, 64, 2048), (1924, 96, 2048), (2048, 132, 1924), (1924, 260, 1988), (4100, 60, 964)]
 
 
@@ -24,7 +24,7 @@ def test_every_tile_edge_and_step_count(form):
     rng = np.random.default_rng(form)
     for m, k, n in SHAPES:
         if form == lib.LEFT:
-            k -= 1  # neither operand's rows run along K
+            k += 1 if k < 32 else -1  # neither operand's rows run along K
         a = rng.uniform(-1, 1, (k, m) if form == lib.LEFT else (m, k)).astype(np.float32)
         b = rng.uniform(-1, 1, (n, k) if form == lib.RIGHT else (k, n)).astype(np.float32)
         wa = (a.T if form == lib.LEFT else a).astype(np.float64)
