@@ -58,12 +58,12 @@ HEADLINE_TRAFFIC = 1.751e9
 # their algorithmic bytes.
 MEASURED_TRAFFIC = {
     "f16 GEMM 16384x1024x4096": 3.419e+08,
-    "f32 GEMM 4096x4096x4096": 6.041e+08,
+    "f32 GEMM 4096x4096x4096": 8.562e+08,
     "x*y, f32 [256,512,512] x [1,512,1]": 5.364e+08,
     "t+z, f32 [256,512,512] + [256,1,512]": 5.406e+08,
     "permute(0,2,1).contiguous, f32 [256,512,512]": 5.364e+08,
     "slice [:,128:384,:].contiguous, f32": 2.682e+08,
-    "concat of two [256,256,512] halves on axis 1, f32": 5.366e+08,
+    "concat of two [256,256,512] halves on axis 1, f32": 5.364e+08,
     "same-shape add, f32 64 Mi elements": 8.048e+08,
     "sum_axes [2] of f32 [64x128x1024]": 3.366e+07,
     "var_axes [2] of f32 [64x128x1024]": 3.366e+07,
@@ -80,13 +80,13 @@ MEASURED_TRAFFIC = {
     "dot, f32 64 Mi elements": 5.37e+08,
     "transpose, f32 [4096x4096]": 1.342e+08,
     "layer norm f32 [8192x8192] (fused_with_statistics), statistics and program in one kernel": 5.368e+08,
-    "layer norm f32 [8192x8192] (fused_with_statistics), composed: row moments, then the program": 8.059e+08,
+    "layer norm f32 [8192x8192] (fused_with_statistics), composed: row moments, then the program": 8.072e+08,
     "Adam update, 25175040 f32 parameters (fused program)": 7.043e+08,
-    "MLP training step 1024-4096-4096-1024, batch 4096, f32, tape + Adam (configs[4])": 8.402e+09,
+    "MLP training step 1024-4096-4096-1024, batch 4096, f32, tape + Adam (configs[4])": 8.474e+09,
     "bf16 dense layer relu(x w + b) 8192x8192x8192, in the product's epilogue": 1.752e+09,
-    "bf16 dense layer relu(x w + b) 8192x8192x8192, unfused: product, then program": 2.318e+09,
-    "f32 dense layer relu(x w + b) 4096x1024x4096, in the product's epilogue": 2.015e+08,
-    "f32 dense layer relu(x w + b) 4096x1024x4096, unfused: product, then program": 3.356e+08,
+    "bf16 dense layer relu(x w + b) 8192x8192x8192, unfused: product, then program": 2.02e+09,
+    "f32 dense layer relu(x w + b) 4096x1024x4096, in the product's epilogue": 2.463e+08,
+    "f32 dense layer relu(x w + b) 4096x1024x4096, unfused: product, then program": 3.739e+08,
 }
 MFMA_PEAK = {"bf16": 2516.6, "f16": 2516.6, "f32": 157.3}  # dense TFLOP/s
 KIND = {"bf16": lib.BF16, "f16": lib.F16, "f32": lib.F32}

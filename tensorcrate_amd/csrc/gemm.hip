@@ -8,15 +8,16 @@
 // matrix cores', not the host's left-to-right FMA chain, so results agree
 // with the host within the f32 tolerance the reference's Metal products keep.
 //
-// 16-bit operands (the tiled kernel below, v_mfma_f32_32x32x16_{bf16,f16})
-// are read in whatever orientation they are stored in: a K-contiguous
-// operand's LDS tile is read with ds_read_b128, a row-contiguous one's with
-// gfx950's transposing ds_read_tr16_b64, so `matmul`, `matmul_add` and both
-// `matmul_transposed_add` forms run the same kernel with no transpose pass.
-// Blocks own 256 x 256 tiles of C over eight waves (128 x 128 over four for
-// small products) and walk K 64 at a time.  HBM reaches LDS through buffer
-// loads that write LDS directly (no staging registers), into XOR-swizzled,
-// double-buffered tiles; out-of-range reads return zeros.  Each step's loads,
+// 16-bit operands (the tiled kernels of gemm_kernels.hpp) are read in whatever
+// orientation they are stored in: a K-contiguous operand's LDS tile is read with
+// ds_read_b128, a row-contiguous one's with gfx950's transposing
+// ds_read_tr16_b64, so `matmul`, `matmul_add` and both `matmul_transposed_add`
+// forms run the same kernel with no transpose pass.
+// Blocks own 256 x 256 tiles of C over eight waves or four (128 x 128 or 128 x 64
+// over four where those are fewer than the CUs) and walk K 64 at a time.  HBM
+// reaches LDS through buffer loads that write LDS directly (no staging
+// registers), into XOR-swizzled tiles of two stages (three or four where a block
+// has its CU to itself); out-of-range reads return zeros.  Each step's loads,
 // LDS reads and matrix-core steps are woven with scheduling groups, and the
 // step's barrier sits before its last slice so the next step's first
 // fragments are read under that slice's matrix-core steps.
