@@ -393,9 +393,8 @@ __global__ void __launch_bounds__(256) rows_kernel(const S* __restrict__ in, O* 
             const I packs = count / V;
             // Whole rounds for all of the slice's lanes, then the rest for all
             // of them, so that no lane runs one part while another waits.
-            const I rounds = packs / (lanes * U);
-            I p = at;
-            for (I k = 0; k < rounds; k++, p += lanes * U) {
+            I p = at, rest = packs;
+            for (; rest >= lanes * U; rest -= lanes * U, p += lanes * U) {
                 float x[U * V];
                 load_packs<S, U, NT, false, I>(slice, p, lanes, 0, x);
                 P::template add_packs<U, V>(s, x, static_cast<uint32_t>(begin + p * V), static_cast<uint32_t>(lanes * V));
@@ -409,9 +408,9 @@ __global__ void __launch_bounds__(256) rows_kernel(const S* __restrict__ in, O* 
                 P::template add_some<R, V>(s, x, left, static_cast<uint32_t>(begin + p * V),
                                            static_cast<uint32_t>(lanes * V));
             };
-            if (!P::kLight && packs - rounds * lanes * U <= lanes) {
+            if (!P::kLight && rest <= lanes) {
                 add_rest(std::integral_constant<int, 1>{});
-            } else if (!P::kLight && packs - rounds * lanes * U <= lanes * 2) {
+            } else if (!P::kLight && rest <= lanes * 2) {
                 add_rest(std::integral_constant<int, 2>{});
             } else {
                 add_rest(std::integral_constant<int, U>{});
